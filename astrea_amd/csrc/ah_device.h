@@ -14,6 +14,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace ah {
 
 enum { EDGE = 0, WRAP = 1 };
@@ -71,9 +73,78 @@ __device__ inline float ah_fabs(float x) { return ::fabsf(x); }
 __device__ inline bool ah_isfinite(double x) { return __builtin_isfinite(x); }
 __device__ inline bool ah_isfinite(float x) { return __builtin_isfinite(x); }
 
+// ---- FP64 in a known range ----------------------------------------------------
+// A double whose divisions and square roots skip the range handling of the
+// general expansions.  The compiler's FP64 division scales both operands,
+// refines v_rcp_f64 by two Newton steps, corrects the quotient and undoes the
+// scaling (17 issue slots of 4 cycles on gfx950, two of them the 8-cycle
+// v_div_scale_f64 and one the 8-cycle v_div_fmas_f64); its square root scales
+// and classifies around v_rsq_f64 with two residual corrections (23 slots).
+// With operands and results far from the ends of the exponent range the
+// scalings are by one, so the refinement alone gives the same bits: 11 slots a
+// division (3 when the divisor's reciprocal is already there -- the sequence
+// is plain arithmetic on the divisor, which the compiler shares between
+// quotients), 14 a square root, and no branch between independent chains.
+// Callers establish the range first (safe_states) and keep the general
+// arithmetic for everything outside it; within it no operand is a NaN or an
+// infinity, so minima and maxima are the hardware's.
+struct fd {
+    double v;
+    fd() = default;
+    __device__ constexpr explicit fd(double x) : v(x) {}
+    __device__ explicit operator double() const { return v; }
+    __device__ friend fd operator+(fd a, fd b) { return fd(a.v + b.v); }
+    __device__ friend fd operator-(fd a, fd b) { return fd(a.v - b.v); }
+    __device__ friend fd operator*(fd a, fd b) { return fd(a.v * b.v); }
+    __device__ friend fd operator-(fd a) { return fd(-a.v); }
+    __device__ friend fd operator/(fd a, fd b) {
+        double r = __builtin_amdgcn_rcp(b.v);
+        r = __builtin_fma(r, __builtin_fma(-b.v, r, 1.0), r);
+        r = __builtin_fma(r, __builtin_fma(-b.v, r, 1.0), r);
+        const double q = a.v * r;
+        return fd(__builtin_fma(__builtin_fma(-b.v, q, a.v), r, q));
+    }
+    __device__ friend bool operator<(fd a, fd b) { return a.v < b.v; }
+    __device__ friend bool operator>(fd a, fd b) { return a.v > b.v; }
+    __device__ friend bool operator<=(fd a, fd b) { return a.v <= b.v; }
+    __device__ friend bool operator>=(fd a, fd b) { return a.v >= b.v; }
+    __device__ friend bool operator==(fd a, fd b) { return a.v == b.v; }
+    __device__ friend bool operator!=(fd a, fd b) { return a.v != b.v; }
+};
+template <class R>
+inline constexpr bool is_fd = sizeof(R) == sizeof(fd) && !std::is_floating_point<R>::value;
+
+__device__ inline fd ah_sqrt(fd x) {
+    // 2^-1000 changes no operand but a zero, for which the chain then gives zero
+    const double y = __builtin_amdgcn_rsq(x.v + 0x1p-1000);
+    double g = x.v * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(g, r, g);
+    g = __builtin_fma(__builtin_fma(-g, g, x.v), h, g);
+    return fd(__builtin_fma(__builtin_fma(-g, g, x.v), h, g));
+}
+__device__ inline fd ah_fabs(fd x) { return fd(::fabs(x.v)); }
+__device__ inline bool ah_isfinite(fd x) { return __builtin_isfinite(x.v); }
+
 // ---- elementary operations (functions/fv.py:19-38) --------------------------
+__device__ inline fd gdiv(fd a, fd b) {
+    const fd q = a / b;
+    return b.v != 0.0 ? q : fd(0.0);
+}
+// fv.divide by a sum or product of densities and sound speeds: positive in
+// fd's range, so that no zero has to be looked for
+template <class R>
+__device__ inline R gdiv_pos(R a, R b);
+__device__ inline fd nmin(fd a, fd b) { return fd(__builtin_fmin(a.v, b.v)); }
+__device__ inline fd nmax(fd a, fd b) { return fd(__builtin_fmax(a.v, b.v)); }
 template <class R>
 __device__ inline R gdiv(R a, R b) { return b != R(0) ? a / b : R(0); }   // fv.divide
+template <class R>
+__device__ inline R gdiv_pos(R a, R b) {
+    if constexpr (is_fd<R>) return a / b;
+    else return gdiv(a, b);
+}
 template <class R>
 __device__ inline R nmin(R a, R b) { return (a < b || a != a) ? a : b; }  // np.minimum (NaN-propagating)
 template <class R>
@@ -156,6 +227,34 @@ __device__ inline R dot_vB(const V8<R>& w) {
     return acc;
 }
 
+// Whether the arithmetic of fd is exact on what the hydrodynamic solvers form
+// from two primitive states: density and pressure in [2^-60, 2^60], velocities
+// zero or in [2^-100, 2^60].  Differences and averages of such values are zero
+// or at least 2^-210, wave speeds and their differences zero or at least
+// 2^-440, the numerators of the HLLC speeds zero or at least 2^-703 and their
+// quotients at most 2^900: every remainder a division or square root corrects
+// with is a normal number (>= 2^-969 before the correction).
+template <int MASK>
+__device__ inline bool safe_states(const V8<double>& a, const V8<double>& b) {
+    using V = VS<MASK>;
+    double sum = (a.c[0] + b.c[0]) + (a.c[4] + b.c[4]);  // NaN and infinities fail the comparison
+    int ex = 0;
+#pragma unroll
+    for (int i = 1; i < 4; ++i)
+        if (V::live(i)) {
+            sum = sum + (ah_fabs(a.c[i]) + ah_fabs(b.c[i]));
+            const int ea = __builtin_amdgcn_frexp_exp(a.c[i]), eb = __builtin_amdgcn_frexp_exp(b.c[i]);
+            ex = min(ex, min(ea, eb));  // 0 for a zero
+        }
+    const double low = __builtin_fmin(__builtin_fmin(a.c[0], b.c[0]), __builtin_fmin(a.c[4], b.c[4]));
+    return sum <= 0x1p60 && low >= 0x1p-60 && ex >= -99;
+}
+// the same for states derived from safe ones (averages, transverse corrections)
+template <class R>
+__device__ inline bool safe_derived(const V8<R>& a, const V8<R>& b) {
+    return __builtin_fmin(__builtin_fmin(a.c[0], b.c[0]), __builtin_fmin(a.c[4], b.c[4])) > 0.0;
+}
+
 // ---- variable conversions (fv.py:49-54, 89-101) ------------------------------
 template <class R, int MASK>
 __device__ inline V8<R> prim_to_cons(const V8<R>& w, R gamma) {
@@ -223,11 +322,11 @@ __device__ inline V8<R> roe_avg(const V8<R>& wp, const V8<R>& wm) {
     a.c[0] = rm * rp;
 #pragma unroll
     for (int i = 1; i < 4; ++i)
-        if (V::live(i)) a.c[i] = gdiv(wp.c[i] * rp + wm.c[i] * rm, s);
-    a.c[4] = gdiv(rp * wp.c[4] + rm * wm.c[4], s);
+        if (V::live(i)) a.c[i] = gdiv_pos(wp.c[i] * rp + wm.c[i] * rm, s);
+    a.c[4] = gdiv_pos(rp * wp.c[4] + rm * wm.c[4], s);
 #pragma unroll
     for (int i = 5; i < 8; ++i)
-        if (V::live(i)) a.c[i] = gdiv(wp.c[i] * rm + wm.c[i] * rp, s);
+        if (V::live(i)) a.c[i] = gdiv_pos(wp.c[i] * rm + wm.c[i] * rp, s);
     return a;
 }
 template <class R, int MASK>
@@ -247,12 +346,13 @@ __device__ inline V8<R> arith_avg(const V8<R>& wp, const V8<R>& wm) {
 template <class R, int MASK, int AX>
 __device__ inline R spectral_radius(const V8<R>& w, R gamma) {
     using V = VS<MASK>;
+    const R rho = w.c[0], u = w.c[AX + 1], p = w.c[4];
+    const R a2 = gamma * p / rho;
+    if constexpr (is_fd<R> && !V::MHD) return ah_fabs(u) + ah_sqrt(a2);  // finite, p > 0
     bool fin = true;
 #pragma unroll
     for (int i = 0; i < 8; ++i)
         if (V::live(i)) fin = fin && ah_isfinite(w.c[i]);
-    const R rho = w.c[0], u = w.c[AX + 1], p = w.c[4];
-    const R a2 = gamma * p / rho;
     R r;
     if constexpr (!V::MHD) {
         r = a2 >= R(0) ? ah_fabs(u) + ah_sqrt(a2) : ah_sqrt(ah_fabs(u * u - a2));
@@ -436,45 +536,73 @@ __device__ inline R lw_coef(const V8<R>& w, R r, R gamma) {
 // HLLC (solvers.py:92-138).  sax = the solver's axis argument (the
 // enumeration index of the sweep, solvers.py:34-36); the reference writes the
 // star momentum at index 1 whatever the axis (127-128), `mom` selects it.
+// The flux is formed in two parts: hllc_wave holds the divisions and roots and
+// reads the primitive states only, hllc_flux assembles the selected flux.
+template <class R>
+struct HllcWave {
+    R k, sS;    // star factor (sS - u) / (sS - sM) and outer speed of the selected side
+    R mom, en;  // rho k sM, and the energy's k (sM - u) (rho sM + p / (sS - u))
+    int sel;    // 1: F*L, 2: F*R, 3: F(w+), 0: default
+};
+
 template <class R, int MASK>
-__device__ inline V8<R> flux_hllc(const Iface<R>& s, int sax, R gamma, int mom, bool default_minus) {
+__device__ inline HllcWave<R> hllc_wave(const V8<R>& wm, const V8<R>& wp, int sax, R gamma) {
     using V = VS<MASK>;
-    const R rhoL = s.wm.c[0], pL = s.wm.c[4], rhoR = s.wp.c[0], pR = s.wp.c[4];
-    const R uL = sax == 0 ? s.wm.c[1] : (V::live(2) ? s.wm.c[2] : R(0));
-    const R uR = sax == 0 ? s.wp.c[1] : (V::live(2) ? s.wp.c[2] : R(0));
-    const R cL = ah_sqrt(gamma * gdiv(pL, rhoL)), cR = ah_sqrt(gamma * gdiv(pR, rhoR));
+    const R rhoL = wm.c[0], pL = wm.c[4], rhoR = wp.c[0], pR = wp.c[4];
+    const R uL = sax == 0 ? wm.c[1] : (V::live(2) ? wm.c[2] : R(0));
+    const R uR = sax == 0 ? wp.c[1] : (V::live(2) ? wp.c[2] : R(0));
+    const R cL = ah_sqrt(gamma * gdiv_pos(pL, rhoL)), cR = ah_sqrt(gamma * gdiv_pos(pR, rhoR));
     const R sqL = ah_sqrt(rhoL), sqR = ah_sqrt(rhoR);
     const R ssum = sqL + sqR;
-    const R u_hat = gdiv(uL * sqL + uR * sqR, ssum);
-    const R c2_hat = gdiv(sqL * (cL * cL) + sqR * (cR * cR), ssum) + R(0.5) * sq(uR - uL) * gdiv(sqL * sqR, ssum * ssum);
+    const R u_hat = gdiv_pos(uL * sqL + uR * sqR, ssum);
+    const R c2_hat = gdiv_pos(sqL * (cL * cL) + sqR * (cR * cR), ssum) + R(0.5) * sq(uR - uL) * gdiv_pos(sqL * sqR, ssum * ssum);
     const R sc = ah_sqrt(c2_hat);
     const R sL = nmin(uL - cL, u_hat - sc);
     const R sR = nmax(uR + cR, u_hat + sc);
     const R sM = gdiv(pR - pL + rhoL * uL * (sL - uL) - rhoR * uR * (sR - uR), rhoL * (sL - uL) - rhoR * (sR - uR));
-    const R kL = gdiv(sL - uL, sL - sM), kR = gdiv(sR - uR, sR - sM);
     const bool useL = (sL <= R(0)) && (R(0) < sM);
     const bool useR = (sM <= R(0)) && (R(0) <= sR);
     const bool useP = sR < R(0);
-    // select first, then evaluate one star flux: F(w+) | F*L | F*R | default.
-    // The reference's default is F(w+) (solvers.py:133), which is the
-    // downwind flux when all waves move right; `default_minus` gives F(w-).
-    if (useP) return s.fp;
-    if (!(useL || useR)) return default_minus ? s.fm : s.fp;
-    V8<R> F = s.fp;
+    // select first, then evaluate one star flux
     const bool left = useL && !useR;
-    const V8<R>& Q = left ? s.qm : s.qp;
-    const V8<R>& Fb = left ? s.fm : s.fp;
-    const R k = left ? kL : kR, rho = left ? rhoL : rhoR, u = left ? uL : uR, p = left ? pL : pR;
+    const R rho = left ? rhoL : rhoR, u = left ? uL : uR, p = left ? pL : pR;
     const R sS = left ? sL : sR;
+    const R k = gdiv(sS - u, sS - sM);
+    HllcWave<R> h;
+    h.k = k;
+    h.sS = sS;
+    h.mom = rho * k * sM;
+    h.en = k * (sM - u) * (rho * sM + gdiv(p, sS - u));
+    h.sel = useP ? 3 : (useR ? 2 : (useL ? 1 : 0));
+    return h;
+}
+
+// F(w+) | F*L | F*R | default from the face's q and f.  The reference's default
+// is F(w+) (solvers.py:133), which is the downwind flux when all waves move
+// right; `default_minus` gives F(w-).
+template <class R, int MASK>
+__device__ inline V8<R> hllc_flux(const HllcWave<R>& h, const V8<R>& qm, const V8<R>& qp, const V8<R>& fm,
+                                  const V8<R>& fp, int mom, bool default_minus) {
+    using V = VS<MASK>;
+    V8<R> F = zero8<R, MASK>();
+    const bool left = h.sel == 1, star = left || h.sel == 2;
+    const bool minus = left || (h.sel == 0 && default_minus);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         if (!V::live(i)) continue;
-        R qs = Q.c[i] * k;
-        if (i == mom) qs = rho * k * sM;
-        if (i == 4) qs = qs + k * (sM - u) * (rho * sM + gdiv(p, sS - u));
-        F.c[i] = Fb.c[i] + (qs - Q.c[i]) * sS;
+        const R Q = left ? qm.c[i] : qp.c[i], f = minus ? fm.c[i] : fp.c[i];
+        R qs = Q * h.k;
+        if (i == mom) qs = h.mom;
+        if (i == 4) qs = qs + h.en;
+        const R g = f + (qs - Q) * h.sS;
+        F.c[i] = star ? g : f;
     }
     return F;
+}
+
+template <class R, int MASK>
+__device__ inline V8<R> flux_hllc(const Iface<R>& s, int sax, R gamma, int mom, bool default_minus) {
+    return hllc_flux<R, MASK>(hllc_wave<R, MASK>(s.wm, s.wp, sax, gamma), s.qm, s.qp, s.fm, s.fp, mom, default_minus);
 }
 
 // A value the whole workgroup shares, read from lane 0 so that the compiler
