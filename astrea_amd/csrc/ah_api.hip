@@ -74,6 +74,52 @@ bool author_supported(const ah_scheme* sch) {
            !sch->magnetic_2d && !sch->fuse2d && sch->tile_s == 0;
 }
 
+// Lines per tile of the marching flux launch, or 0 for the 2D flux tiles.
+//
+// A marching wave solves its own lines and two halo lines one after another,
+// so a launch takes about (rounds of resident waves) x (lines + 2) line times:
+// long tiles waste less on halo lines, short ones fill the chip.  The lines
+// are those with the least of that product; past two rounds the waves drain
+// unevenly and half a round is added for the tail.  Two hydrodynamic waves
+// (256 registers) or one MHD wave (394) fit a SIMD.
+//
+// Below some cells the launch is one round of a few lines whatever they are,
+// and the tiles, whose four waves share one line's latency, end sooner.
+// Measured, us per launch (x + y sweep), tiles against marching: PPM/HLLC
+// 384^2 48 / 51, 512^2 63 / 62, 640^2 88 / 79, 1024^2 208 / 133; WENO5/LLF
+// 517 x 333 44 / 41, 512^2 PLM 52 / 45, 384^2 37 / 36; PLM/HLLD 384^2 87 / 82,
+// 512^2 124 / 110, 256^2 42 / 64.
+int march_lines_for(const ah_scheme& sch, int nprob, const ah_problem* probs, int cus, KernelSet* ks) {
+    if (sch.precision != AH_FP64 || sch.fuse2d || sch.ppm_author != AH_PPM_MC) return 0;
+    long long cells = 0;
+    for (int i = 0; i < nprob; ++i) {
+        if (probs[i].n0 <= 0 || probs[i].n1 <= 0) return 0;
+        cells += (long long)probs[i].n0 * probs[i].n1;
+    }
+    if (cells < (sch.solver == AH_LLF ? 160000 : 250000)) return 0;
+    if (!kernels_2d_march_fp64(sch.varmask, sch.recon, sch.solver, ks)) return 0;
+    const double slots = (ks->march_waves * 4) * (double)cus;
+    int best = 0;
+    double best_cost = 0.0;
+    for (int lines = 3; lines <= 24; ++lines) {
+        double cost = 0.0;
+        for (int ax = 0; ax < 2; ++ax) {
+            double waves = 0.0;
+            for (int i = 0; i < nprob; ++i) {
+                const int ns = ax == 0 ? probs[i].n0 : probs[i].n1, nt = ax == 0 ? probs[i].n1 : probs[i].n0;
+                waves += (double)((ns + ks->mw - 1) / ks->mw) * ((nt + lines - 1) / lines);
+            }
+            const double rounds = waves / slots;
+            cost += (rounds <= 2.0 ? (rounds <= 1.0 ? 1.0 : 2.0) : rounds + .5) * (lines + 2);
+        }
+        if (best == 0 || cost < best_cost) {
+            best = lines;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
 int popcount8(int m) {
     int n = 0;
     for (int c = 0; c < 8; ++c) n += (m >> c) & 1;
@@ -292,6 +338,11 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
         delete p;
         return AH_ERR_UNSUPPORTED;
     }
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) == hipSuccess) {
+        hipDeviceProp_t prop;
+        if (hipGetDeviceProperties(&prop, dev) == hipSuccess) cus = prop.multiProcessorCount;
+    }
     // registers: K1..K4 (1-4), saved L (5-8)
     switch (sch->rk) {
         case AH_EULER: p->nregs = 0; break;
@@ -303,6 +354,10 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
         case AH_SSPRK54: p->nregs = 5; break;
         case AH_SSPRK104: p->nregs = sch->magnetic_2d ? 4 : 3; break;  // + the refined increment
     }
+    // the marching flux launch where it is the faster form
+    const int march_lines = sch->dims == 2 ? march_lines_for(p->sch, nprob, probs, cus, &p->ks) : 0;
+    if (march_lines > 0)
+        for (int ax = 0; ax < 2; ++ax) p->ks.flux[ax] = p->ks.march[ax];
     // problem tables and tiles
     std::vector<ProbDesc> pd(nprob);
     long long max_ctiles = 0;
@@ -336,8 +391,18 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
                 if (p->ks.recon[ax])  // no reconstruction launch when the flux tiles reconstruct
                     for (int t0 = 0; t0 < nt; t0 += p->ks.rtt[ax])
                         for (int s0 = 0; s0 < ns; s0 += p->ks.rts[ax]) p->tl[1 + ax].full.push_back({i, s0, t0, 0});
-                for (int t0 = 0; t0 < nt; t0 += p->ks.ftt[ax])
-                    for (int s0 = 0; s0 < ns; s0 += p->ks.fts[ax]) p->tl[3 + ax].full.push_back({i, s0, t0, 0});
+                if (march_lines > 0) {
+                    // even splits: no tile is left with a few cells or lines
+                    const int nw = (ns + p->ks.mw - 1) / p->ks.mw, nl = (nt + march_lines - 1) / march_lines;
+                    for (int l = 0; l < nl; ++l)
+                        for (int w = 0; w < nw; ++w) {
+                            const int sb = (int)((long long)ns * w / nw), se = (int)((long long)ns * (w + 1) / nw);
+                            const int tb = (int)((long long)nt * l / nl), te = (int)((long long)nt * (l + 1) / nl);
+                            p->tl[3 + ax].full.push_back({i, sb, tb, march_pad(se - sb, te - tb)});
+                        }
+                } else
+                    for (int t0 = 0; t0 < nt; t0 += p->ks.ftt[ax])
+                        for (int s0 = 0; s0 < ns; s0 += p->ks.fts[ax]) p->tl[3 + ax].full.push_back({i, s0, t0, 0});
                 if (sch->magnetic_2d)
                     for (int t0 = 0; t0 < nt; t0 += p->ks.ttt)
                         for (int s0 = 0; s0 < ns; s0 += p->ks.tts) p->tl[6 + ax].full.push_back({i, s0, t0, 0});
@@ -376,11 +441,6 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
         if (up && L.count)
             up = hipMalloc((void**)&L.d, L.full.size() * sizeof(Tile)) == hipSuccess &&
                  hipMemcpy(L.d, L.full.data(), L.full.size() * sizeof(Tile), hipMemcpyHostToDevice) == hipSuccess;
-    }
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        hipDeviceProp_t prop;
-        if (hipGetDeviceProperties(&prop, dev) == hipSuccess) cus = prop.multiProcessorCount;
     }
     // 32 workgroups per CU: a 1024^2 grid's sweeps then launch one workgroup
     // per tile and the hardware balances the last round (2048 persistent

@@ -169,6 +169,26 @@ inline void set2d_author(KernelSet* ks) {
     };
 }
 
+// The 2D flux launches in marching form (FP64; LLF, HLLC, HLLD on point or
+// 4th-order face conversion), beside the tile form; the plan picks one
+template <int MASK, int SOLVER, int CONV>
+inline bool set2d_march(KernelSet* ks) {
+    ks->march[0] = [](const SweepArgs& a, int nb, hipStream_t s) {
+        launch_sweep(flux2d_march_kernel<MASK, SOLVER, CONV, 0>, a, nb, s, 64);
+    };
+    ks->march[1] = [](const SweepArgs& a, int nb, hipStream_t s) {
+        launch_sweep(flux2d_march_kernel<MASK, SOLVER, CONV, 1>, a, nb, s, 64);
+    };
+    ks->mw = march_width<SOLVER>();
+    ks->march_waves = march_waves<MASK>();
+    return true;
+}
+
+template <int MASK, int SOLVER>
+inline bool set2d_march(int recon, KernelSet* ks) {
+    return recon == PCM ? false : (recon == PLM ? set2d_march<MASK, SOLVER, 1>(ks) : set2d_march<MASK, SOLVER, 2>(ks));
+}
+
 // 2D hydrodynamics, one launch per sweep: the flux kernel reconstructs its
 // own window (recon[] stays null, and the plan keeps no wL/wR planes).  The
 // 16 x 8 tile takes 52 KB of LDS (the reconstruction windows share theirs

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "ah_march.h"
 #include "ah_mhd.h"
 
 namespace ah {
@@ -17,6 +18,11 @@ struct KernelSet {
     SweepLaunch sweep1d = nullptr;
     SweepLaunch recon[2] = {nullptr, nullptr};
     SweepLaunch flux[2] = {nullptr, nullptr};
+    // the flux launch in marching form (null where only the tile form exists)
+    // with its own cells per tile along the sweep
+    SweepLaunch march[2] = {nullptr, nullptr};
+    int mw = 0;
+    int march_waves = 1;  // resident waves per SIMD
     int ts1 = 0;
     int rts[2] = {0, 0}, rtt[2] = {0, 0};
     int fts[2] = {0, 0}, ftt[2] = {0, 0};
@@ -39,6 +45,9 @@ bool kernels_1d_small_fp32(int mask, int recon, int solver, KernelSet* ks);
 // 1D / 2D hydrodynamic PPM with author c (1) or ph (2), FP64, LLF or HLLC
 bool kernels_1d_author_fp64(int author, int solver, KernelSet* ks);
 bool kernels_2d_author_fp64(int author, int solver, KernelSet* ks);
+// adds the marching flux launchers (false: the combination has the tile form only)
+bool kernels_2d_march_fp64(int mask, int recon, int solver, KernelSet* ks);
+bool kernels_2d_march_mhd_fp64(int mask, int recon, int solver, KernelSet* ks);
 bool kernels_2d_fp32(int mask, int recon, int solver, KernelSet* ks);
 // 2D hydrodynamic PLM/PPM with LLF or HLLC, one launch per sweep (recon[] null)
 bool kernels_2d_fused_fp64(int recon, int solver, KernelSet* ks);

@@ -5,8 +5,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def _grid(shape, seed):
-    """Conservative hydrodynamic state of order one with jumps, gas at rest and smooth parts."""
+def _grid(shape, seed, mhd=False):
+    """Conservative state of order one with jumps, gas at rest and smooth parts (and a field)."""
     r = np.random.default_rng(seed)
     n = int(np.prod(shape))
     w = np.zeros((n, 8))
@@ -17,6 +17,9 @@ def _grid(shape, seed):
         v = np.where(r.random(n) < .3, 0., r.uniform(-1.5, 1.5, n))
         w[:, c] = rho * v
         w[:, 4] += .5 * rho * v * v
+    for c in (5, 6) if mhd else ():
+        w[:, c] = .4 + .2 * r.random(n)
+        w[:, 4] += .5 * w[:, c] ** 2
     return w.reshape(shape + (8,))
 
 
@@ -55,3 +58,55 @@ def test_short_divisions_and_roots_give_the_general_bits(shape, solver, subgrid,
                 want = np.ldexp(ref[q][ax]["flux"][..., :5], [s + c for s in scale])
                 assert np.array_equal(got[q][ax]["flux"][..., :5], want), (a, c, q, ax)
                 assert got[q][ax]["eigmax"] == np.ldexp(ref[q][ax]["eigmax"], c)
+
+
+@pytest.mark.parametrize("shape", [(512, 513), (126, 2050), (2, 130000), (4000, 63), (64, 4100)], ids=str)
+@pytest.mark.parametrize("subgrid,solver,boundary", [("ppm", "hllc", "wrap"), ("plm", "hllc", "edge"),
+                                                     ("weno5", "llf", "edge")])
+def test_marching_flux_equals_the_tiles(shape, subgrid, solver, boundary):
+    """Fluxes and eigmax of a plan large enough for the marching flux launch
+    against the allocation-free entry point, which runs the 2D tiles: sides
+    that are one tile wide, one more, one less, shorter than a stencil."""
+    import torch
+    from astrea_amd.plan import Plan
+    from tests.test_zz_no_alloc import _static_call
+    plan = Plan(2, subgrid, solver, "ssprk(3,3)",
+                [dict(n0=shape[0], n1=shape[1], boundary=boundary, dx=1 / 512, gamma=1.4, cfl=.4, t_end=1e9)],
+                varmask=0x17)
+    plan.load([torch.from_numpy(_grid(shape, 5)).cuda()])
+    for parity in (0, 1):
+        ref = plan.evolve_space(parity)
+        rc, f0, f1, eig = _static_call(plan, parity)
+        assert rc == 0
+        assert torch.equal(f0, ref[0]["raw"]) and torch.equal(f1, ref[1]["raw"])
+        assert eig == [ref[0]["eigmax"], ref[1]["eigmax"]]
+    plan.close()
+
+
+@pytest.mark.parametrize("subgrid,solver,timestep,boundary,mhd", [
+    ("ppm", "hllc", "ssprk(3,3)", "edge", False), ("plm", "llf", "rk4", "wrap", False),
+    ("weno5", "hlld", "ssprk(3,3)", "wrap", True), ("ppm", "hlld", "rk4", "edge", True)])
+def test_marching_batch_equals_its_problems_alone(subgrid, solver, timestep, boundary, mhd):
+    """Three steps of a ragged batch, large enough together for the marching
+    launch, against each problem alone on the 2D tiles, bit for bit."""
+    import torch
+    from astrea_amd.plan import Plan
+    shapes = [(5, 7), (64, 63), (62, 126), (2, 9), (130, 33), (77, 205), (63, 64), (200, 3), (455, 480)]
+    probs = [dict(n0=a, n1=b, boundary=boundary, dx=1 / max(a, b), gamma=1.4, cfl=.3, t_end=1e9) for a, b in shapes]
+    grids = [torch.from_numpy(_grid(s, 11 + i, mhd)).cuda() for i, s in enumerate(shapes)]
+
+    def run(ps, gs):
+        plan = Plan(2, subgrid, solver, timestep, ps, varmask=0x77 if mhd else 0x17, magnetic_2d=mhd,
+                    compat="physical")
+        plan.load(gs)
+        plan.reset()
+        plan.step(3)
+        out, st = plan.state.clone(), plan.status()
+        offs = plan.offsets + [plan.total]
+        plan.close()
+        return [out[:, offs[i]:offs[i + 1]] for i in range(len(ps))], st
+    both, st = run(probs, grids)
+    for i in range(len(shapes)):
+        (one,), (s1,) = run(probs[i:i + 1], grids[i:i + 1])
+        assert torch.equal(torch.nan_to_num(both[i]), torch.nan_to_num(one)), shapes[i]
+        assert st[i] == s1, shapes[i]
