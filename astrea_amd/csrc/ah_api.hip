@@ -148,6 +148,7 @@ struct ah_plan {
     ProbDesc* d_pd = nullptr;
     ProbState* d_ps = nullptr;
     unsigned* d_done = nullptr;  // per problem: tiles of the step's last combination done
+    int comb_cells = 256;        // cells per combination tile
     bool fold_finish = false;    // the last combination ends the step (few tiles per problem)
     // tile lists: 0 = 1D sweep, 1/2 = recon ax0/ax1, 3/4 = flux ax0/ax1, 5 = cells (combine),
     // 6/7 = transverse reconstruction ax0/ax1 (MHD)
@@ -360,6 +361,13 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
         for (int ax = 0; ax < 2; ++ax) p->ks.flux[ax] = p->ks.march[ax];
     // problem tables and tiles
     std::vector<ProbDesc> pd(nprob);
+    // combination tiles: 256 cells (one per thread) in 1D, so the few large
+    // problems left at the end of an ensemble still spread over many CUs, and
+    // in 2D up to 128^2, whose 64 tiles still end the step themselves (below);
+    // 1024 beyond, where four cells per thread ran faster on 1024^2 grids
+    long long most_cells = 0;
+    for (int i = 0; i < nprob; ++i) most_cells = std::max(most_cells, (long long)probs[i].n0 * std::max(probs[i].n1, 1));
+    p->comb_cells = sch->dims == 1 || most_cells <= 64 * 256 ? 256 : 1024;
     long long max_ctiles = 0;
     long long total = 0;
     for (int i = 0; i < nprob; ++i) {
@@ -408,10 +416,7 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
                         for (int s0 = 0; s0 < ns; s0 += p->ks.tts) p->tl[6 + ax].full.push_back({i, s0, t0, 0});
             }
         }
-        // combination tiles: 256 cells (one per thread) in 1D, so the few large
-        // problems left at the end of an ensemble still spread over many CUs;
-        // 1024 in 2D, where four cells per thread ran faster on 1024^2 grids
-        const int ct = sch->dims == 1 ? 256 : 1024;
+        const int ct = p->comb_cells;
         for (long long c0 = 0; c0 < cells; c0 += ct)
             p->tl[5].full.push_back({i, (int)c0, (int)std::min<long long>(ct, cells - c0), 0});
         max_ctiles = std::max(max_ctiles, (cells + ct - 1) / ct);
@@ -667,7 +672,7 @@ static void launch_space(ah_plan* p, const double* X, double* Lout, int stage0, 
 static void launch_combine(ah_plan* p, int op, hipStream_t s, bool stored_dt = false, bool finish = false) {
     CombineArgs c;
     c.finish = finish ? 1 : 0;
-    c.ct = p->sch.dims == 1 ? 256 : 1024;
+    c.ct = p->comb_cells;
     c.done = p->d_done;
     c.live_dt = (p->sch.magnetic_2d || stored_dt) ? 0 : 1;
     c.dims = p->sch.dims;
@@ -679,22 +684,8 @@ static void launch_combine(ah_plan* p, int op, hipStream_t s, bool stored_dt = f
     c.ntiles_dev = p->tl[5].d_count;
     c.plane = p->total;
     c.nv = p->nv;
-    c.op = op;
     ProfScope ps_(p, AH_K_COMBINE, s);
-    hipLaunchKernelGGL(combine_kernel, dim3(blocks_for(p, p->tl[5])), dim3(256), 0, s, c);
-}
-
-// register each stage combination writes (for the MHD refinement)
-static int target_reg(int op) {
-    switch (op) {
-        case OP_EULER: case OP_22_1: case OP_33_2: case OP_43_3: case OP_RK4_3: case OP_53_4: case OP_54_4:
-        case OP_104_FINAL: return 0;
-        case OP_22_0: case OP_33_0: case OP_43_0: case OP_RK4_0: case OP_53_0: case OP_54_0: return 1;
-        case OP_33_1: case OP_43_1: case OP_RK4_1: case OP_53_1: case OP_54_1: return 2;
-        case OP_43_2: case OP_RK4_2: case OP_53_2: case OP_54_2: case OP_104_K5: return 3;
-        case OP_53_3: case OP_54_3: return 4;
-    }
-    return -1;
+    combine_launcher(op, p->comb_cells > 256)(c, blocks_for(p, p->tl[5]), s);
 }
 
 // SSPRK(10,4) stages that add a refined increment: the addition that
@@ -730,7 +721,7 @@ static void combine_refine(ah_plan* p, int op, hipStream_t s, bool stored_dt = f
         return;
     }
     launch_combine(p, op, s, stored_dt);
-    double* K = p->regs[target_reg(op)];
+    double* K = p->regs[rk_writes(op)];
     m.K = K;
     p->ks.refine(m, blocks_for(p, p->tl[7]), s);
     p->ks.copyB(m, K, blocks_for(p, p->tl[5]), s);

@@ -4,6 +4,8 @@
 #pragma once
 #include "ah_kernels.h"
 
+#include <utility>
+
 namespace ah {
 
 // ============================================================================
@@ -145,7 +147,6 @@ struct CombineArgs {
     const int* ntiles_dev;
     long long plane;
     int nv;
-    int op;
     int live_dt;   // 1: dt from step_dt (no dt launch in this step program), 0: the stored dt
     int dims;
     // finish: this combination ends the step, and the block that combines a
@@ -157,86 +158,158 @@ struct CombineArgs {
     unsigned* done;
 };
 
+// registers an operation reads (bit r: regs[r]), the one it writes, and the
+// one it saves the stage's L in (-1: none)
+constexpr int rk_reads(int op) {
+    constexpr int U = 1, K1 = 2, K2 = 4, K3 = 8, K4 = 16, L5 = 32, L6 = 64, L7 = 128;
+    switch (op) {
+        case OP_22_1: case OP_33_1: return U | K1;
+        case OP_33_2: return U | K2;
+        case OP_43_1: case OP_53_1: return K1;
+        case OP_43_2: return U | K2;
+        case OP_43_3: return K3;
+        case OP_RK4_3: return U | L5 | L6 | L7;
+        case OP_53_2: return U | K2;
+        case OP_53_3: return U | K1 | K3 | L5;
+        case OP_53_4: return U | K1 | K2 | K4 | L5 | L6;
+        case OP_54_1: return U | K1;
+        case OP_54_2: return U | K2;
+        case OP_54_3: return U | K3;
+        case OP_54_4: return K2 | K3 | K4 | L5;
+        case OP_104_ACC1: return K1;
+        case OP_104_K5: return U | K1;
+        case OP_104_K2FIRST: return K3;
+        case OP_104_ACC2: return K2;
+        case OP_104_INC: return 0;
+        case OP_104_ADD_U: return U | K4;
+        case OP_104_ADD_K1: return K1 | K4;
+        case OP_104_ADD_K3: return K3 | K4;
+        case OP_104_ADD_K2: return K2 | K4;
+        case OP_104_FINAL: return U | K3 | K2;
+    }
+    return U;
+}
+constexpr int rk_writes(int op) {
+    switch (op) {
+        case OP_22_0: case OP_33_0: case OP_43_0: case OP_RK4_0: case OP_53_0: case OP_54_0: case OP_104_FIRST:
+        case OP_104_ACC1: case OP_104_ADD_U: case OP_104_ADD_K1: return 1;
+        case OP_33_1: case OP_43_1: case OP_RK4_1: case OP_53_1: case OP_54_1: case OP_104_K2FIRST: case OP_104_ACC2:
+        case OP_104_ADD_K3: case OP_104_ADD_K2: return 2;
+        case OP_43_2: case OP_RK4_2: case OP_53_2: case OP_54_2: case OP_104_K5: return 3;
+        case OP_53_3: case OP_54_3: case OP_104_INC: return 4;
+    }
+    return 0;
+}
+constexpr int rk_saves(int op) {
+    switch (op) {
+        case OP_RK4_0: case OP_53_0: case OP_54_3: return 5;
+        case OP_RK4_1: case OP_53_1: return 6;
+        case OP_RK4_2: return 7;
+    }
+    return -1;
+}
+constexpr int RK_OPS = OP_104_ADD_K2 + 1;
+
+// one value, from the registers' values r, the stage's L and dt
+template <int OP>
+__device__ inline double rk_value(const double (&r)[9], double L, double dt) {
+    const double U = r[0], K1 = r[1], K2 = r[2], K3 = r[3], K4 = r[4];
+    switch (OP) {
+        case OP_EULER: return U + dt * L;
+        case OP_22_0: return U + dt * L;
+        case OP_22_1: return .5 * (U + K1 + dt * L);
+        case OP_33_0: return U + dt * L;
+        case OP_33_1: return .25 * (3 * U + K1 + dt * L);
+        case OP_33_2: return (1.0 / 3.0) * (U + 2 * K2 + 2 * dt * L);
+        case OP_43_0: return U + .5 * dt * L;
+        case OP_43_1: return K1 + .5 * dt * L;
+        case OP_43_2: return (1.0 / 6.0) * (4 * U + 2 * K2 + dt * L);
+        case OP_43_3: return K3 + .5 * dt * L;
+        case OP_RK4_0: return U + .5 * dt * L;
+        case OP_RK4_1: return U + .5 * dt * L;
+        case OP_RK4_2: return U + dt * L;
+        case OP_RK4_3: return U + (1.0 / 6.0) * (dt * (r[5] + 2 * r[6] + 2 * r[7] + L));
+        case OP_53_0: return U + .3772689151171 * dt * L;
+        case OP_53_1: return K1 + .3772689151171 * dt * L;
+        case OP_53_2: return .56656131914033 * U + .43343868085967 * K2 + .16352294089771 * dt * L;
+        case OP_53_3:
+            return .09299483444413 * U + .0000209036962 * K1 + .90698426185967 * K3 + .00071997378654 * dt * r[5] +
+                   .34217696850008 * dt * L;
+        case OP_53_4:
+            return .0073613226092 * U + .20127980325145 * K1 + .00182955389682 * K2 + .78952932024253 * K4 +
+                   (dt * (.0027771981946 * r[5] + .00001567934613 * r[6] + .29786487010104 * L));
+        case OP_54_0: return U + .39175222657189 * dt * L;
+        case OP_54_1: return .444370493651235 * U + .555629506348765 * K1 + .368410593050371 * dt * L;
+        case OP_54_2: return .620101851488403 * U + .379898148511597 * K2 + .251891774271694 * dt * L;
+        case OP_54_3: return .178079954393132 * U + .821920045606868 * K3 + .544974750228521 * dt * L;
+        case OP_54_4:
+            return .517231671970585 * K2 + .096059710526147 * K3 + .06369246866629 * dt * r[5] +
+                   .386708617503269 * K4 + .226007483236906 * dt * L;
+        case OP_104_FIRST: return U + (1.0 / 6.0) * dt * L;
+        case OP_104_ACC1: return K1 + (1.0 / 6.0) * dt * L;
+        case OP_104_K5: return 3.0 / 5.0 * U + 6.0 / 15.0 * K1 + 1.0 / 15.0 * dt * L;
+        case OP_104_K2FIRST: return K3 + (1.0 / 6.0) * dt * L;
+        case OP_104_ACC2: return K2 + (1.0 / 6.0) * dt * L;
+        case OP_104_INC: return (1.0 / 6.0) * dt * L;
+        case OP_104_ADD_U: return U + K4;
+        case OP_104_ADD_K1: return K1 + K4;
+        case OP_104_ADD_K3: return K3 + K4;
+        case OP_104_ADD_K2: return K2 + K4;
+        case OP_104_FINAL: return -11.0 / 35.0 * U + 5.0 / 7.0 * K3 + 3.0 / 5.0 * K2 + 1.0 / 10.0 * dt * L;
+    }
+    return 0.0;
+}
+
+// Four values per thread and turn: the next four components of one cell on
+// tiles of 256 cells, four cells of one component on tiles of 1024.  All their
+// loads leave before the first value is formed: the kernel is bound by memory
+// bandwidth on large grids and by the length of its chain of loads on small
+// ones (one value after another, a 128^2 tile of 4 x 4 values per thread took
+// 12 us).  The tile's descriptor, the problem's and its time state are each
+// read whole, so that the branch on the state costs one round trip, not four.
+template <int OP, bool WIDE>
 __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
     const long long n = a.plane;
     const int ntiles = wave_uniform(*a.ntiles_dev);
     for (int ti = blockIdx.x; ti < ntiles; ti += gridDim.x) {
         const Tile tl = ld_const(a.tiles + ti);
-        const ProbState& s = a.ps[tl.prob];
-        if (!ld_const(&s.active)) continue;
-        if (!ld_const(&s.fail_flag)) {
-        double dt;
-        if (a.live_dt) {
+        const ProbState s = ld_const(a.ps + tl.prob);
+        const ProbDesc d = ld_const(a.pd + tl.prob);
+        if (!s.active) continue;
+        if (!s.fail_flag) {
             int hit;
-            dt = step_dt(ld_const(&a.pd[tl.prob]), s, a.dims, &hit);
-        } else {
-            dt = ld_const(&s.dt);
-        }
-        const long long base = ld_const(&a.pd[tl.prob].off) + tl.s0;
-        for (int c = threadIdx.x; c < tl.t0; c += blockDim.x)
-        for (int v = 0; v < a.nv; ++v) {
-            const long long j = v * n + base + c;
-            double* U = a.regs[0];
-            double* K1 = a.regs[1];
-            double* K2 = a.regs[2];
-            double* K3 = a.regs[3];
-            double* K4 = a.regs[4];
-            const double L = a.L[j];
-            switch (a.op) {
-                case OP_EULER: U[j] = U[j] + dt * L; break;
-                case OP_22_0: K1[j] = U[j] + dt * L; break;
-                case OP_22_1: U[j] = .5 * (U[j] + K1[j] + dt * L); break;
-                case OP_33_0: K1[j] = U[j] + dt * L; break;
-                case OP_33_1: K2[j] = .25 * (3 * U[j] + K1[j] + dt * L); break;
-                case OP_33_2: U[j] = (1.0 / 3.0) * (U[j] + 2 * K2[j] + 2 * dt * L); break;
-                case OP_43_0: K1[j] = U[j] + .5 * dt * L; break;
-                case OP_43_1: K2[j] = K1[j] + .5 * dt * L; break;
-                case OP_43_2: K3[j] = (1.0 / 6.0) * (4 * U[j] + 2 * K2[j] + dt * L); break;
-                case OP_43_3: U[j] = K3[j] + .5 * dt * L; break;
-                case OP_RK4_0: a.regs[5][j] = L; K1[j] = U[j] + .5 * dt * L; break;
-                case OP_RK4_1: a.regs[6][j] = L; K2[j] = U[j] + .5 * dt * L; break;
-                case OP_RK4_2: a.regs[7][j] = L; K3[j] = U[j] + dt * L; break;
-                case OP_RK4_3:
-                    U[j] = U[j] + (1.0 / 6.0) * (dt * (a.regs[5][j] + 2 * a.regs[6][j] + 2 * a.regs[7][j] + L));
-                    break;
-                case OP_53_0: a.regs[5][j] = L; K1[j] = U[j] + .3772689151171 * dt * L; break;
-                case OP_53_1: a.regs[6][j] = L; K2[j] = K1[j] + .3772689151171 * dt * L; break;
-                case OP_53_2: K3[j] = .56656131914033 * U[j] + .43343868085967 * K2[j] + .16352294089771 * dt * L; break;
-                case OP_53_3:
-                    K4[j] = .09299483444413 * U[j] + .0000209036962 * K1[j] + .90698426185967 * K3[j] +
-                            .00071997378654 * dt * a.regs[5][j] + .34217696850008 * dt * L;
-                    break;
-                case OP_53_4:
-                    U[j] = .0073613226092 * U[j] + .20127980325145 * K1[j] + .00182955389682 * K2[j] +
-                           .78952932024253 * K4[j] +
-                           (dt * (.0027771981946 * a.regs[5][j] + .00001567934613 * a.regs[6][j] + .29786487010104 * L));
-                    break;
-                case OP_54_0: K1[j] = U[j] + .39175222657189 * dt * L; break;
-                case OP_54_1: K2[j] = .444370493651235 * U[j] + .555629506348765 * K1[j] + .368410593050371 * dt * L; break;
-                case OP_54_2: K3[j] = .620101851488403 * U[j] + .379898148511597 * K2[j] + .251891774271694 * dt * L; break;
-                case OP_54_3:
-                    a.regs[5][j] = L;
-                    K4[j] = .178079954393132 * U[j] + .821920045606868 * K3[j] + .544974750228521 * dt * L;
-                    break;
-                case OP_54_4:
-                    U[j] = .517231671970585 * K2[j] + .096059710526147 * K3[j] + .06369246866629 * dt * a.regs[5][j] +
-                           .386708617503269 * K4[j] + .226007483236906 * dt * L;
-                    break;
-                case OP_104_FIRST: K1[j] = U[j] + (1.0 / 6.0) * dt * L; break;
-                case OP_104_ACC1: K1[j] = K1[j] + (1.0 / 6.0) * dt * L; break;
-                case OP_104_K5: K3[j] = 3.0 / 5.0 * U[j] + 6.0 / 15.0 * K1[j] + 1.0 / 15.0 * dt * L; break;
-                case OP_104_K2FIRST: K2[j] = K3[j] + (1.0 / 6.0) * dt * L; break;
-                case OP_104_ACC2: K2[j] = K2[j] + (1.0 / 6.0) * dt * L; break;
-                case OP_104_INC: K4[j] = (1.0 / 6.0) * dt * L; break;
-                case OP_104_ADD_U: K1[j] = U[j] + K4[j]; break;
-                case OP_104_ADD_K1: K1[j] = K1[j] + K4[j]; break;
-                case OP_104_ADD_K3: K2[j] = K3[j] + K4[j]; break;
-                case OP_104_ADD_K2: K2[j] = K2[j] + K4[j]; break;
-                case OP_104_FINAL:
-                    U[j] = -11.0 / 35.0 * U[j] + 5.0 / 7.0 * K3[j] + 3.0 / 5.0 * K2[j] + 1.0 / 10.0 * dt * L;
-                    break;
+            const double dt = a.live_dt ? step_dt(d, s, a.dims, &hit) : s.dt;
+            const long long base = d.off + tl.s0;
+            auto four = [&](int v0, int dv, int c0, int dc) {
+                double r[4][9], L[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int v = v0 + u * dv, c = c0 + u * dc;
+                    if (v < a.nv && c < tl.t0) {
+                        const long long j = v * n + base + c;
+                        L[u] = a.L[j];
+#pragma unroll
+                        for (int k = 0; k < 8; ++k)
+                            if ((rk_reads(OP) >> k) & 1) r[u][k] = a.regs[k][j];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int v = v0 + u * dv, c = c0 + u * dc;
+                    if (v < a.nv && c < tl.t0) {
+                        const long long j = v * n + base + c;
+                        if constexpr (rk_saves(OP) >= 0) a.regs[rk_saves(OP)][j] = L[u];
+                        a.regs[rk_writes(OP)][j] = rk_value<OP>(r[u], L[u], dt);
+                    }
+                }
+            };
+            if constexpr (WIDE) {
+                for (int v = 0; v < a.nv; ++v)
+                    for (int c = threadIdx.x; c < tl.t0; c += 4 * 256) four(v, 0, c, 256);
+            } else {
+                for (int c = threadIdx.x; c < tl.t0; c += 256)
+                    for (int v = 0; v < a.nv; v += 4) four(v, 1, c, 0);
             }
-        }
         }
         if (a.finish) {
             // every block that combines one of the problem's tiles counts it
@@ -247,7 +320,6 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
             // launch sees it.
             __syncthreads();
             if (threadIdx.x == 0) {
-                const ProbDesc d = ld_const(&a.pd[tl.prob]);
                 const long long cells = (long long)d.n0 * d.n1;
                 const unsigned nt = (unsigned)((cells + a.ct - 1) / a.ct);
                 if (atomicAdd(&a.done[tl.prob], 1u) == nt - 1) {
@@ -259,6 +331,19 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
     }
 }
 
+
+using CombineLaunch = void (*)(const CombineArgs&, int nblocks, hipStream_t);
+template <bool WIDE, int... OP>
+inline CombineLaunch combine_launcher(int op, std::integer_sequence<int, OP...>) {
+    static constexpr CombineLaunch table[] = {[](const CombineArgs& a, int nb, hipStream_t s) {
+        hipLaunchKernelGGL((combine_kernel<OP, WIDE>), dim3(nb), dim3(256), 0, s, a);
+    }...};
+    return table[op];
+}
+inline CombineLaunch combine_launcher(int op, bool wide) {
+    using Ops = std::make_integer_sequence<int, RK_OPS>;
+    return wide ? combine_launcher<true>(op, Ops()) : combine_launcher<false>(op, Ops());
+}
 
 // L = -sum_a dF_a/dx from sweep-frame interface fluxes (evolvers.py:41-60)
 __global__ void fluxdiff_kernel(const double* F0, const double* F1, double* L, int n0, int n1, int dims, int nv,

@@ -85,10 +85,16 @@ def test_marching_flux_equals_the_tiles(shape, subgrid, solver, boundary):
 
 @pytest.mark.parametrize("subgrid,solver,timestep,boundary,mhd", [
     ("ppm", "hllc", "ssprk(3,3)", "edge", False), ("plm", "llf", "rk4", "wrap", False),
-    ("weno5", "hlld", "ssprk(3,3)", "wrap", True), ("ppm", "hlld", "rk4", "edge", True)])
+    ("weno5", "hlld", "ssprk(3,3)", "wrap", True), ("ppm", "hlld", "rk4", "edge", True),
+    ("plm", "hllc", "euler", "edge", False), ("plm", "hllc", "ssprk(2,2)", "edge", False),
+    ("plm", "llf", "ssprk(4,3)", "edge", False), ("plm", "llf", "ssprk(5,3)", "wrap", False),
+    ("ppm", "hllc", "ssprk(5,4)", "wrap", False), ("plm", "hllc", "ssprk(10,4)", "edge", False),
+    ("plm", "hlld", "ssprk(10,4)", "wrap", True)])
 def test_marching_batch_equals_its_problems_alone(subgrid, solver, timestep, boundary, mhd):
     """Three steps of a ragged batch, large enough together for the marching
-    launch, against each problem alone on the 2D tiles, bit for bit."""
+    launch and the 1024-cell combination tiles, against each problem alone on
+    the 2D tiles (and, but for the largest, 256-cell combination tiles), bit
+    for bit."""
     import torch
     from astrea_amd.plan import Plan
     shapes = [(5, 7), (64, 63), (62, 126), (2, 9), (130, 33), (77, 205), (63, 64), (200, 3), (455, 480)]
