@@ -226,8 +226,11 @@ void launch_snapshot(const ah_plan* p, int prob, double* out, hipStream_t s, con
     const int bc = q.boundary == AH_WRAP ? WRAP : EDGE;
     const bool ho = p->sch.recon == AH_PPM || p->sch.recon == AH_WENO3 || p->sch.recon == AH_WENO5 ||
                     p->sch.recon == AH_WENO7;
-    const long long cells = (long long)q.n0 * n1;
-    const dim3 g((unsigned)((cells + 255) / 256)), b(256);
+    // the kernel's tiles (256 cells in 1D)
+    const long long tiles = p->sch.dims == 1
+                                ? (q.n0 + 255) / 256
+                                : (long long)((q.n0 + SNAP_TI - 1) / SNAP_TI) * ((n1 + SNAP_TJ - 1) / SNAP_TJ);
+    const dim3 g((unsigned)tiles), b(256);
     const long long off = p->offs[prob];
     if (p->sch.dims == 1) {
         if (ho) hipLaunchKernelGGL((snapshot_kernel<MASK, 1, true>), g, b, 0, s, p->U, p->total, off, q.n0, n1, bc, q.gamma, out, cap);

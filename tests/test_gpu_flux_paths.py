@@ -116,3 +116,30 @@ def test_marching_batch_equals_its_problems_alone(subgrid, solver, timestep, bou
         (one,), (s1,) = run(probs[i:i + 1], grids[i:i + 1])
         assert torch.equal(torch.nan_to_num(both[i]), torch.nan_to_num(one)), shapes[i]
         assert st[i] == s1, shapes[i]
+
+
+@pytest.mark.parametrize("shape", [(1,), (255,), (257,), (8, 32), (9, 31), (7, 33), (1, 70), (50, 2)], ids=str)
+@pytest.mark.parametrize("subgrid,boundary", [("ppm", "wrap"), ("ppm", "edge"), ("plm", "edge")])
+def test_snapshot_at_tile_edges_and_unaligned_buffers(shape, subgrid, boundary):
+    """The snapshot of grids around one tile of the conversion kernel, into a
+    16-byte aligned buffer and into one that is not, against the oracle's
+    conversion of the same state."""
+    import torch
+    from astrea_amd.plan import Plan
+    from oracle import astrea_oracle as O
+    dims = len(shape)
+    g = _grid(shape, 9)
+    plan = Plan(dims, subgrid, "llf", "euler",
+                [dict(n0=shape[0], n1=shape[1] if dims == 2 else 1, boundary=boundary, dx=.1, gamma=1.4, cfl=.4,
+                      t_end=1.)], varmask=0x13 if dims == 1 else 0x17)
+    plan.load([g])
+    s = O.Scheme(dimension=dims, subgrid=subgrid, boundary=boundary, gamma=1.4, dx=.1)
+    w = O.to_prim(g, s)
+    want = w if dims == 1 else np.ascontiguousarray(w.transpose(1, 0, 2))
+    n = int(np.prod(shape)) * 8
+    for skip in (0, 1):
+        buf = torch.full((n + 2,), np.nan, dtype=torch.float64, device="cuda")
+        out = buf[skip:skip + n].view(shape[::-1] + (8,))
+        assert np.array_equal(plan.snapshot(0, out=out).cpu().numpy(), want)
+        assert bool(torch.isnan(buf[:skip]).all()) and bool(torch.isnan(buf[skip + n:]).all())
+    plan.close()
