@@ -136,8 +136,8 @@ __device__ inline fd gdiv(fd a, fd b) {
 // fd's range, so that no zero has to be looked for
 template <class R>
 __device__ inline R gdiv_pos(R a, R b);
-__device__ inline fd nmin(fd a, fd b) { return fd(__builtin_fmin(a.v, b.v)); }
-__device__ inline fd nmax(fd a, fd b) { return fd(__builtin_fmax(a.v, b.v)); }
+__device__ inline fd nmin(fd a, fd b);
+__device__ inline fd nmax(fd a, fd b);
 template <class R>
 __device__ inline R gdiv(R a, R b) { return b != R(0) ? a / b : R(0); }   // fv.divide
 template <class R>
@@ -179,6 +179,37 @@ __device__ inline double hmin(double a, double b) { return __builtin_fmin(a, b);
 __device__ inline float hmin(float a, float b) { return __builtin_fminf(a, b); }
 __device__ inline double hmax(double a, double b) { return __builtin_fmax(a, b); }
 __device__ inline float hmax(float a, float b) { return __builtin_fmaxf(a, b); }
+// The instructions themselves, plain and of absolute values: the compiler's
+// fmin/fmax first quiet each operand it has not just computed, one more
+// instruction apiece.
+__device__ inline double imin(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ inline double imax(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ inline double imin_abs(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ inline double imax_abs(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ inline float imin(float a, float b) { return hmin(a, b); }
+__device__ inline float imax(float a, float b) { return hmax(a, b); }
+__device__ inline float imin_abs(float a, float b) { return hmin(ah_fabs(a), ah_fabs(b)); }
+__device__ inline float imax_abs(float a, float b) { return hmax(ah_fabs(a), ah_fabs(b)); }
+__device__ inline double ah_copysign(double m, double s) { return __builtin_copysign(m, s); }
+__device__ inline float ah_copysign(float m, float s) { return __builtin_copysignf(m, s); }
+__device__ inline fd nmin(fd a, fd b) { return fd(imin(a.v, b.v)); }
+__device__ inline fd nmax(fd a, fd b) { return fd(imax(a.v, b.v)); }
 template <class R>
 __device__ inline R sq(R x) { return x * x; }
 
@@ -395,6 +426,7 @@ __device__ inline R slope_limit(int lim, R a, R b) {
 // cell extremum), so only that branch exists here.
 // Inputs: wS, neighbours wm1/wp1/wm2/wp2, face values fL/fR, curvatures
 // d2 at i-1, i, i+1 and third differences d3 at i-2..i+2.
+// The branches pay: most waves lie in uniform or smooth regions and skip them.
 template <class R>
 __device__ inline void mc_limit(R wS, R wm1, R wp1, R wm2, R wp2, R fL, R fR, R d2m, R d2c, R d2p, R d3m2, R d3m1,
                                 R d30, R d3p2, R& wL, R& wR) {
@@ -404,16 +436,16 @@ __device__ inline void mc_limit(R wS, R wm1, R wp1, R wm2, R wp2, R fL, R fR, R 
     wR = fR;
     const R d2w = R(6) * (fL - R(2) * wS + fR);
     const bool cell_extrema = (dwm * dwp <= R(0)) || ((wS - wm2) * (wp2 - wS) <= R(0));
-    // min/max over absolute values: no negative zeros (hmin/hmax exact)
-    const R lim_curv = nsign(d2c) * hmin(hmin(ah_fabs(d2w), C * ah_fabs(d2c)), hmin(C * ah_fabs(d2p), C * ah_fabs(d2m)));
+    // min/max over absolute values: no negative zeros (imin/imax exact)
+    const R lim_curv = nsign(d2c) * imin(imin_abs(d2w, C * d2c), imin_abs(C * d2p, C * d2m));
     const R d2w_lim = cell_extrema ? lim_curv : R(0);
-    const bool sens = ah_fabs(d2w) > R(1e-12) * hmax(ah_fabs(wS), hmax(hmax(ah_fabs(wm1), ah_fabs(wp1)), hmax(ah_fabs(wm2), ah_fabs(wp2))));
+    const bool sens = ah_fabs(d2w) > R(1e-12) * imax_abs(wS, imax(imax_abs(wm1, wp1), imax_abs(wm2, wp2)));
     const R rho = sens ? gdiv(d2w_lim, d2w) : R(0);
     // d3min/d3max enter only through |.| and d3max - d3min, which compare
     // the same against 0.1 max(|d3max|, |d3min|) whatever the zeros' signs
-    const R d3min = hmin(hmin(d3m1, d30), hmin(d3m2, d3p2));
-    const R d3max = hmax(hmax(d3m1, d30), hmax(d3m2, d3p2));
-    const bool roundoff = (rho < R(1.0 - 1e-12)) || (R(0.1) * hmax(ah_fabs(d3max), ah_fabs(d3min)) <= (d3max - d3min));
+    const R d3min = imin(imin(d3m1, d30), imin(d3m2, d3p2));
+    const R d3max = imax(imax(d3m1, d30), imax(d3m2, d3p2));
+    const bool roundoff = (rho < R(1.0 - 1e-12)) || (R(0.1) * imax_abs(d3max, d3min) <= (d3max - d3min));
     if ((dwm * dwp < R(0)) && roundoff) {
         wL = wS - rho * dwm;
         wR = wS + rho * dwp;

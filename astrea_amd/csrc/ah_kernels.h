@@ -880,10 +880,16 @@ struct RowAcc {
 // sweep-frame layout [t][s] (s contiguous) of type R.
 // ============================================================================
 // Hydrodynamic tiles take 39 KB of LDS, room for four workgroups per CU; the
-// register budget is capped so that four waves fit each SIMD (the PPM
-// instantiations spill 80 bytes per lane to do so and still run 10 % faster
-// than at three waves on the 1024^2 shear layer).  MHD windows leave LDS for
-// three, so their registers stay uncapped.
+// register budget is capped so that four waves fit each SIMD.  MHD windows
+// leave LDS for three, so their registers stay uncapped.
+// PPM in FP64 is bound by instruction issue and LDS reads, so the faces and
+// curvatures that neighbouring cells share are formed once per position and
+// kept where the dead conversion windows were (a cell on its own forms two
+// faces and six curvatures).  Per launch, each cell for itself -> shared, x / y:
+// 1024^2 edge 60.7/63.1 -> 49.4/47.6 us, 256^2 13.3/13.2 -> 11.3/11.0, MHD 768^2
+// 58.8/58.1 -> 50.5/48.2, 1024^2 periodic with flattener 54.2/53.2 -> 54.7/53.5
+// (there the flattener's chains bound it).  Split precision keeps the cell
+// form: its contracted rounding has to be the fused kernel's.
 // AUTH (PPM, 2D hydrodynamics, FP64): author 'c' or 'ph' (ppm.py:43-71).  A
 // first launch with flags_only records the stage's grid-wide interface-limiter
 // tests of this sweep (limiters.py:58) in the problem's aflags, bits
@@ -899,8 +905,19 @@ void recon2d_kernel(SweepArgs a) {
     constexpr int NQS = NWS + 2;             // q window  [s0-5, s0+TS+5)
     constexpr int HT = HO ? 1 : 0;           // q rows    [t0-HT, t0+TT+HT)
     constexpr int NQT = TT + 2 * HT;
-    __shared__ double qd[NV][NQT][NQS];
-    __shared__ double cq[HO ? NV : 1][HO ? NQT : 1][HO ? NQS : 1];
+    // q and its primitive form, dead once wS is formed; PPM then keeps each
+    // row's face values (positions [s0-1, s0+TS)) and curvatures
+    // ([s0-2, s0+TS+3)) in their place
+    constexpr bool TWO = RECON == PPM && AUTH == AUTH_MC && !SPLIT;
+    constexpr int NFC = TS + 1, ND2 = TS + 5;
+    constexpr int NQ_ = NV * NQT * NQS, NC2_ = TWO ? NV * TT * (NFC + ND2) : 0;
+    constexpr int NBUF = (HO ? 2 : 1) * NQ_ > NC2_ ? (HO ? 2 : 1) * NQ_ : NC2_;
+    __shared__ double qbuf[NBUF];
+    const auto qd = reinterpret_cast<double (*)[NQT][NQS]>(qbuf);
+    const auto cq = reinterpret_cast<double (*)[NQT][NQS]>(qbuf + (HO ? NQ_ : 0));
+    const auto fc_s = reinterpret_cast<R (*)[TT][NFC]>(qbuf);
+    const auto d2_s = reinterpret_cast<R (*)[TT][ND2]>(qbuf + (TWO ? NV * TT * NFC : 0));
+    static_assert(sizeof(R) == 8, "the windows share one array of doubles");
     __shared__ R ws[NV][TT][NWS];
     // PPM flattener: chi~ of each own row at positions [s0-2, s0+TS]
     constexpr int NCHI = TS + 3;
@@ -1035,16 +1052,60 @@ void recon2d_kernel(SweepArgs a) {
             __syncthreads();
         }
     }
+    if constexpr (TWO) {
+        // Face values and curvatures, once per position (a cell reads two of
+        // the first and six of the second), each evaluated at e(p)
+        for (int i = threadIdx.x; i < TT * ND2; i += blockDim.x) {
+            const int it = i / ND2, j = i % ND2, p = s0 - 2 + j;
+            const RowAcc<R, MASK, TT, NWS, CL> W{ws, it, bws, ns};
+            const int me = W.e(p);
+            const V8<R> wa = W(me - 1), wz = W(me), wb = W(me + 1);
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+                if (V::live(c)) d2_s[V::slot(c)][it][j] = wa.c[c] - R(2) * wz.c[c] + wb.c[c];
+            if (j < 1 || j > NFC) continue;
+            const V8<R> wc = W(me + 2);
+            R eta = R(1);
+            if (a.flattener != FLAT_OFF) {
+                // eta = min(chi(me), chi(me -/+ 1)) by sign of the pressure jump (ppm.py:127-131)
+                auto chi_at = [&](int mm) { return chi_s[it][mm - (s0 - 2)]; };
+                eta = chi_at(me);
+                const R sg = nsign(wb.c[4] - wa.c[4]);
+                const R lo = chi_at(me - 1), hi = chi_at(me + 1);
+                if (sg < R(0)) eta = nmin(eta, hi);
+                if (sg > R(0)) eta = nmin(eta, lo);
+            }
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                if (!V::live(c)) continue;
+                // face interpolant (ppm.py:38), blended toward the cell by eta (ppm.py:65-67)
+                R f = R(K7_12) * (wz.c[c] + wb.c[c]) - R(K1_12) * (wa.c[c] + wc.c[c]);
+                if (a.flattener != FLAT_OFF) f = f * eta + wz.c[c] * (R(1) - eta);
+                fc_s[V::slot(c)][it][j - 1] = f;
+            }
+        }
+        __syncthreads();
+    }
     for (int i = threadIdx.x; i < TT * TS; i += blockDim.x) {
         const int it = i / TS, is = i % TS;
         const int s = s0 + is, t = t0 + it;
         if (s >= ns || t >= nt) continue;
         const RowAcc<R, MASK, TT, NWS, CL> W{ws, it, bws, ns};
         V8<R> L, Rr;
-        if constexpr (RECON == PPM)
-            recon_cell<R, MASK, RECON, AX>(W, s, a.limiter, a.flattener, L, Rr,
-                                           [&](int mm) { return chi_s[it][mm - (s0 - 2)]; });
-        else
+        if constexpr (TWO) {
+            L = Rr = zero8<R, MASK>();
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                if (!V::live(c)) continue;
+                const int v = V::slot(c);
+                auto w = [&](int m) { return ws[v][it][W.e(m) - bws]; };
+                auto d2 = [&](int m) { return d2_s[v][it][m - (s0 - 2)]; };
+                // d3w[m] = d2w_C[e(m+1)] - d2w_C[m] (limiters.py:96), padded by two (126-127)
+                auto d3 = [&](int m) { return d2(W.e(m) + 1) - d2(W.e(m)); };
+                mc_limit<R>(w(s), w(s - 1), w(s + 1), w(s - 2), w(s + 2), fc_s[v][it][is], fc_s[v][it][is + 1],
+                            d2(s - 1), d2(s), d2(s + 1), d3(s - 2), d3(s - 1), d3(s), d3(s + 2), L.c[c], Rr.c[c]);
+            }
+        } else
             recon_cell<R, MASK, RECON, AX>(W, s, a.limiter, a.flattener, L, Rr);
         const long long o = fo + (long long)t * ns + s;
 #pragma unroll
