@@ -272,6 +272,57 @@ __device__ inline void recon_cell(const Acc& W, int ce, int limiter, int flatten
                                    [&](int mm) { return flat_chi_at<R, AX>(W, flattener, mm); });
 }
 
+// PPM in two steps, for a line whose cells share their faces.  First one
+// position's curvature and face value, evaluated at e(p) (ppm.py:38, blended
+// toward the cell by eta, ppm.py:65-67): curvatures at d2_at(component, p - pd),
+// faces at fc_at(component, p - pf) for p in [pf, pf + nf)
+template <class R, int MASK, class Acc, class ChiAt, class D2, class FC>
+__device__ inline void ppm_shared_at(const Acc& W, int p, int pd, int pf, int nf, int flattener, const ChiAt& chi_at,
+                                     const D2& d2_at, const FC& fc_at) {
+    using V = VS<MASK>;
+    const int me = W.e(p);
+    const V8<R> wa = W(me - 1), wz = W(me), wb = W(me + 1);
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+        if (V::live(c)) d2_at(V::slot(c), p - pd) = wa.c[c] - R(2) * wz.c[c] + wb.c[c];
+    if (p < pf || p >= pf + nf) return;
+    const V8<R> wc = W(me + 2);
+    R eta = R(1);
+    if (flattener != FLAT_OFF) {
+        // eta = min(chi(me), chi(me -/+ 1)) by sign of the pressure jump (ppm.py:127-131)
+        eta = chi_at(me);
+        const R sg = nsign(wb.c[4] - wa.c[4]);
+        const R lo = chi_at(me - 1), hi = chi_at(me + 1);
+        if (sg < R(0)) eta = nmin(eta, hi);
+        if (sg > R(0)) eta = nmin(eta, lo);
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        if (!V::live(c)) continue;
+        R f = R(K7_12) * (wz.c[c] + wb.c[c]) - R(K1_12) * (wa.c[c] + wc.c[c]);
+        if (flattener != FLAT_OFF) f = f * eta + wz.c[c] * (R(1) - eta);
+        fc_at(V::slot(c), p - pf) = f;
+    }
+}
+// then cell ce's limited extrapolants
+template <class R, int MASK, class Acc, class D2, class FC>
+__device__ inline void ppm_shared_cell(const Acc& W, int ce, int pd, int pf, const D2& d2_at, const FC& fc_at,
+                                       V8<R>& wL, V8<R>& wR) {
+    using V = VS<MASK>;
+    wL = wR = zero8<R, MASK>();
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        if (!V::live(c)) continue;
+        const int v = V::slot(c);
+        auto w = [&](int m) { return W(m).c[c]; };
+        auto d2 = [&](int m) { return d2_at(v, m - pd); };
+        // d3w[m] = d2w_C[e(m+1)] - d2w_C[m] (limiters.py:96), padded by two (126-127)
+        auto d3 = [&](int m) { return d2(W.e(m) + 1) - d2(W.e(m)); };
+        mc_limit<R>(w(ce), w(ce - 1), w(ce + 1), w(ce - 2), w(ce + 2), fc_at(v, ce - 1 - pf), fc_at(v, ce - pf),
+                    d2(ce - 1), d2(ce), d2(ce + 1), d3(ce - 2), d3(ce - 1), d3(ce), d3(ce + 2), wL.c[c], wR.c[c]);
+    }
+}
+
 // ---- PPM authors 'c' and 'ph' (ppm.py:43-62, 69-71) ----------------------------
 // Colella et al. 2011 and Peterson & Hammett 2008: not reachable from the
 // reference's options (evolvers.py:17 passes author 'mc'), built as the
@@ -476,6 +527,13 @@ __device__ inline void block_max_atomic(double v, unsigned long long* dst, doubl
 // 1D: one fused kernel per stage: load -> cons->prim -> reconstruct/limit ->
 // spectral radius -> Riemann -> flux difference -> L = -dF/dx.
 // ============================================================================
+// Many tiles are bound by instruction issue, few by one tile's chain of
+// phases.  PPM therefore forms faces and curvatures once per position, the
+// solvers that need no neighbour's radius form theirs with the flux (one phase
+// and one reading of the states less), and the phases' arrays share their
+// places (38 -> 30 KB of LDS, five workgroups per CU).  192 ragged PPM/HLLC
+// problems 31.6 -> 24.6 us per launch, three large ones 8.9 -> 7.5, one MHD tube
+// of 1601 cells (WENO5/HLLD) 14.6 -> 14.1.
 // Window accessor of the 1D sweep: W(m) is the primitive state at e(m);
 // CLAMP = false when the tile's stencil never leaves the domain or the
 // boundary is periodic (e is then the identity).
@@ -518,13 +576,27 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
     __shared__ R ws[NV][NW];
     __shared__ R wl[RECON == PCM ? 1 : NV][RECON == PCM ? 1 : NC];
     __shared__ R wr[RECON == PCM ? 1 : NV][RECON == PCM ? 1 : NC];
-    __shared__ R rad[NR];
-    __shared__ R fl[NV][NF];
+    // only the Lax-Friedrichs and Lax-Wendroff solvers take a neighbour's radius;
+    // the others' own one is formed with their flux
+    constexpr bool MERGED = RECON != PCM && SOLVER != LLF && SOLVER != LW;
+    __shared__ R rad[MERGED ? 1 : NR];
+    // PPM forms face values of positions [s0-2, s0+TS+2) and curvatures of
+    // [s0-3, s0+TS+5) once per position, in cq and qd; the fluxes take cq's
+    // (PLM: qd's) place when the reconstruction is done
+    constexpr bool TWO = RECON == PPM && AUTH == AUTH_MC && !SPLIT;
+    constexpr int ND2 = TS + 8, NFC = TS + 4;
+    static_assert(!TWO || sizeof(R) == 8, "faces and curvatures lie in arrays of doubles");
+    const auto d2_s = reinterpret_cast<R (*)[NQ]>(qd);
+    const auto fc_s = reinterpret_cast<R (*)[NQ]>(cq);
+    __shared__ R flux_s[RECON == PCM ? NV : 1][RECON == PCM ? NQ : 1];
+    const auto fl = reinterpret_cast<R (*)[NQ]>(RECON == PCM ? (void*)flux_s : HO ? (void*)cq : (void*)qd);
     __shared__ double red[4];
     __shared__ unsigned abits;  // PPM authors c/ph: the tile's interface-limiter tests
     // PPM flattener: chi~ at positions [s0-3, s0+TS+2]
     constexpr int NCHI = TS + 6;
-    __shared__ R chi_s[RECON == PPM ? NCHI : 1];
+    __shared__ R chi_b[RECON == PPM && !TWO ? NCHI : 1];
+    R* const chi_s = TWO ? &wl[0][0] : chi_b;  // read before the first wl is written
+    static_assert(!TWO || NV * NC >= NCHI, "chi~ lies in wl");
 
     const int ntiles_ = wave_uniform(a.ntiles_dev ? *a.ntiles_dev : a.ntiles);
     for (int ti_ = blockIdx.x; ti_ < ntiles_; ti_ += gridDim.x) {
@@ -661,9 +733,21 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
                     __syncthreads();
                 }
             }
+            if constexpr (TWO) {
+                for (int i = threadIdx.x; i < ND2; i += blockDim.x)
+                    ppm_shared_at<R, MASK>(Wc, s0 - 3 + i, s0 - 3, s0 - 2, NFC, a.flattener,
+                                           [&](int mm) { return chi_s[mm - (s0 - 3)]; },
+                                           [&](int v, int j) -> R& { return d2_s[v][j]; },
+                                           [&](int v, int j) -> R& { return fc_s[v][j]; });
+                __syncthreads();
+            }
             for (int i = threadIdx.x; i < NC; i += blockDim.x) {
                 V8<R> L, Rr;
-                if constexpr (RECON == PPM)
+                if constexpr (TWO)
+                    ppm_shared_cell<R, MASK>(Wc, Wc.e(bcl + i), s0 - 3, s0 - 2,
+                                             [&](int v, int j) { return d2_s[v][j]; },
+                                             [&](int v, int j) { return fc_s[v][j]; }, L, Rr);
+                else if constexpr (RECON == PPM)
                     recon_cell<R, MASK, RECON, 0>(Wc, Wc.e(bcl + i), a.limiter, a.flattener, L, Rr,
                                                   [&](int mm) { return chi_s[mm - (s0 - 3)]; });
                 else
@@ -706,10 +790,18 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
         const V8<A> p = cast8<A, R, MASK>(wp), m = cast8<A, R, MASK>(wm);
         return R(spectral_radius<A, MASK, 0>(RECON == PLM ? arith_avg<A, MASK>(p, m) : roe_avg<A, MASK>(p, m), A(gR)));
     };
-    // D: spectral radius of the Jacobian state at padded positions j in [s0, s0+TS+1]
     double lmax = 0.0;
     bool bad = false;
-    for (int i = threadIdx.x; i < NR; i += blockDim.x) {
+    // the step's wave speed over the tile's own interfaces
+    auto own_radius = [&](int j, R r) {
+        if (j >= s0 + 1 && j <= s0 + TS && j >= 1 && j <= N) {
+            const double rd = double(r);
+            if (!(rd <= 1.7976931348623157e308)) bad = true;
+            lmax = (rd > lmax || rd != rd) ? rd : lmax;
+        }
+    };
+    // D: spectral radius of the Jacobian state at padded positions j in [s0, s0+TS+1]
+    if constexpr (!MERGED) for (int i = threadIdx.x; i < NR; i += blockDim.x) {
         const int j = s0 + i;
         V8<R> st;
         R r;
@@ -728,15 +820,13 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
         else if constexpr (!FAST) r = spectral_radius<R, MASK, 0>(st, gR);
         if constexpr (SOLVER == LW) rad[i] = lw_coef<R>(st, r, gR);
         else rad[i] = r;
-        if (j >= s0 + 1 && j <= s0 + TS && j >= 1 && j <= N) {
-            const double rd = double(r);
-            if (!(rd <= 1.7976931348623157e308)) bad = true;
-            lmax = (rd > lmax || rd != rd) ? rd : lmax;
-        }
+        own_radius(j, r);
     }
-    if (bad) atomicOr(&ps->fail_flag, 1);
-    if (a.stage0) block_max_atomic(lmax, &ps->eig[0], red);
-    __syncthreads();
+    if constexpr (!MERGED) {
+        if (bad) atomicOr(&ps->fail_flag, 1);
+        if (a.stage0) block_max_atomic(lmax, &ps->eig[0], red);
+        __syncthreads();
+    }
     // E: interface fluxes k in [s0, s0+TS]
     for (int i = threadIdx.x; i < NF; i += blockDim.x) {
         const int k = s0 + i;
@@ -759,7 +849,8 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
             f.qm = prim_to_cons_split<MASK>(f.wm, gamma);
             f.qp = prim_to_cons_split<MASK>(f.wp, gamma);
         }
-        const R lam = nmax(rad[i], rad[i + 1]);
+        R lam = R(0);
+        if constexpr (!MERGED) lam = nmax(rad[i], rad[i + 1]);
         R Bn = R(0);
         if constexpr (SOLVER == HLLD) Bn = W(e(k)).c[5];
         V8<R> F;
@@ -782,6 +873,10 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
             } else {
                 g.fm = phys_flux<A, MASK, 0>(g.wm, A(gR));
                 g.fp = phys_flux<A, MASK, 0>(g.wp, A(gR));
+            }
+            if constexpr (MERGED) {
+                if constexpr (SPLIT) own_radius(k, radius<MASK, 0, true>(jac_state<MASK, true, RECON != PLM>(f.wp, f.wm), gamma));
+                else own_radius(k, radius_of(arith, f.wp, f.wm));
             }
             F = cast8<R, A, MASK>(riemann<A, MASK, SOLVER, 0>(g, A(lam), sax, A(Bn), A(gR), 1, a.compat != 0, SPLIT));
         };
@@ -810,7 +905,12 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
 #pragma unroll
                     for (int c = 0; c < 8; ++c)
                         if (V::live(c)) {
-                            const R dq = R(qd[V::slot(c)][e(k) - bq] - qd[V::slot(c)][e(k - 1) - bq]);
+                            // (the shared curvatures have taken the window's place)
+                            auto Qc = [&](int m) {
+                                return TWO ? stage_x(a, V::slot(c) * P + off + bcmap(e(m), N, bc), xdt)
+                                           : qd[V::slot(c)][e(m) - bq];
+                            };
+                            const R dq = R(Qc(k) - Qc(k - 1));
                             F.c[c] = F.c[c] + R(0.3) * (nu * dq);
                         }
                 }
@@ -824,6 +924,10 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
             for (int c = 0; c < 8; ++c)
                 if (V::live(c)) a.flux_out[V::slot(c) * a.flux_plane + k] = double(F.c[c]);
         }
+    }
+    if constexpr (MERGED) {
+        if (bad) atomicOr(&ps->fail_flag, 1);
+        if (a.stage0) block_max_atomic(lmax, &ps->eig[0], red);
     }
     __syncthreads();
     // F: L = -(F[i+1] - F[i]) / dx (evolvers.py:41-60)
@@ -1056,33 +1160,12 @@ void recon2d_kernel(SweepArgs a) {
         // Face values and curvatures, once per position (a cell reads two of
         // the first and six of the second), each evaluated at e(p)
         for (int i = threadIdx.x; i < TT * ND2; i += blockDim.x) {
-            const int it = i / ND2, j = i % ND2, p = s0 - 2 + j;
+            const int it = i / ND2, j = i % ND2;
             const RowAcc<R, MASK, TT, NWS, CL> W{ws, it, bws, ns};
-            const int me = W.e(p);
-            const V8<R> wa = W(me - 1), wz = W(me), wb = W(me + 1);
-#pragma unroll
-            for (int c = 0; c < 8; ++c)
-                if (V::live(c)) d2_s[V::slot(c)][it][j] = wa.c[c] - R(2) * wz.c[c] + wb.c[c];
-            if (j < 1 || j > NFC) continue;
-            const V8<R> wc = W(me + 2);
-            R eta = R(1);
-            if (a.flattener != FLAT_OFF) {
-                // eta = min(chi(me), chi(me -/+ 1)) by sign of the pressure jump (ppm.py:127-131)
-                auto chi_at = [&](int mm) { return chi_s[it][mm - (s0 - 2)]; };
-                eta = chi_at(me);
-                const R sg = nsign(wb.c[4] - wa.c[4]);
-                const R lo = chi_at(me - 1), hi = chi_at(me + 1);
-                if (sg < R(0)) eta = nmin(eta, hi);
-                if (sg > R(0)) eta = nmin(eta, lo);
-            }
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                if (!V::live(c)) continue;
-                // face interpolant (ppm.py:38), blended toward the cell by eta (ppm.py:65-67)
-                R f = R(K7_12) * (wz.c[c] + wb.c[c]) - R(K1_12) * (wa.c[c] + wc.c[c]);
-                if (a.flattener != FLAT_OFF) f = f * eta + wz.c[c] * (R(1) - eta);
-                fc_s[V::slot(c)][it][j - 1] = f;
-            }
+            ppm_shared_at<R, MASK>(W, s0 - 2 + j, s0 - 2, s0 - 1, NFC, a.flattener,
+                                   [&](int mm) { return chi_s[it][mm - (s0 - 2)]; },
+                                   [&](int v, int k) -> R& { return d2_s[v][it][k]; },
+                                   [&](int v, int k) -> R& { return fc_s[v][it][k]; });
         }
         __syncthreads();
     }
@@ -1092,20 +1175,10 @@ void recon2d_kernel(SweepArgs a) {
         if (s >= ns || t >= nt) continue;
         const RowAcc<R, MASK, TT, NWS, CL> W{ws, it, bws, ns};
         V8<R> L, Rr;
-        if constexpr (TWO) {
-            L = Rr = zero8<R, MASK>();
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                if (!V::live(c)) continue;
-                const int v = V::slot(c);
-                auto w = [&](int m) { return ws[v][it][W.e(m) - bws]; };
-                auto d2 = [&](int m) { return d2_s[v][it][m - (s0 - 2)]; };
-                // d3w[m] = d2w_C[e(m+1)] - d2w_C[m] (limiters.py:96), padded by two (126-127)
-                auto d3 = [&](int m) { return d2(W.e(m) + 1) - d2(W.e(m)); };
-                mc_limit<R>(w(s), w(s - 1), w(s + 1), w(s - 2), w(s + 2), fc_s[v][it][is], fc_s[v][it][is + 1],
-                            d2(s - 1), d2(s), d2(s + 1), d3(s - 2), d3(s - 1), d3(s), d3(s + 2), L.c[c], Rr.c[c]);
-            }
-        } else
+        if constexpr (TWO)
+            ppm_shared_cell<R, MASK>(W, s, s0 - 2, s0 - 1, [&](int v, int j) { return d2_s[v][it][j]; },
+                                     [&](int v, int j) { return fc_s[v][it][j]; }, L, Rr);
+        else
             recon_cell<R, MASK, RECON, AX>(W, s, a.limiter, a.flattener, L, Rr);
         const long long o = fo + (long long)t * ns + s;
 #pragma unroll

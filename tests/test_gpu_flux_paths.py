@@ -166,3 +166,28 @@ def test_shared_faces_match_each_cell_for_itself(shapes, boundary, flattener):
         plan.close()
     assert torch.equal(torch.nan_to_num(outs[0][0]), torch.nan_to_num(outs[1][0]))
     assert outs[0][1] == outs[1][1]
+
+
+@pytest.mark.parametrize("tile_s", [0, 115])
+@pytest.mark.parametrize("solver,flattener,av", [("hllc", "off", False), ("llf", "astrea", False), ("hllc", "astrea", True)])
+@pytest.mark.parametrize("boundary", ["wrap", "edge"])
+def test_one_dimensional_ppm_around_its_tiles(boundary, solver, flattener, av, tile_s):
+    """1D PPM fluxes and wave speeds of grids around one and two tiles and far
+    below one, against the oracle.  The kernel orders its operations as the
+    oracle does, so only the last bits of a library root or power may differ:
+    1e-14 of the largest flux, some 45 units in the last place."""
+    from astrea_amd.plan import Plan
+    from oracle import astrea_oracle as O
+    for n in (2, 5, 114, 115, 116, 231, 242, 243, 244, 247, 487):
+        g = _grid((n,), 31 + n)
+        plan = Plan(1, "ppm", solver, "ssprk(3,3)",
+                    [dict(n0=n, boundary=boundary, dx=1 / 64, gamma=1.4, cfl=.4, t_end=1e9)], varmask=0x13,
+                    flattener=flattener, av=av, tile_s=tile_s)
+        plan.load([g])
+        got = plan.evolve_space(0)[0]
+        plan.close()
+        s = O.Scheme(dimension=1, subgrid="ppm", solver=solver, boundary=boundary, gamma=1.4, cfl=.4, dx=1 / 64,
+                     flattener=flattener, av=av)
+        want = O.evolve_space(g, s)[0]
+        assert np.abs(got["flux"] - want["flux"]).max() <= 1e-14 * np.abs(want["flux"]).max(), n
+        assert abs(got["eigmax"] - want["eigmax"]) <= 1e-14 * want["eigmax"], n
