@@ -81,7 +81,7 @@ bool author_supported(const ah_scheme* sch) {
 // long tiles waste less on halo lines, short ones fill the chip.  The lines
 // are those with the least of that product; past two rounds the waves drain
 // unevenly and half a round is added for the tail.  Two hydrodynamic waves
-// (256 registers) or one MHD wave (394) fit a SIMD.
+// (256 registers) or one MHD wave (504) fit a SIMD.
 //
 // Below some cells the launch is one round of a few lines whatever they are,
 // and the tiles, whose four waves share one line's latency, end sooner.

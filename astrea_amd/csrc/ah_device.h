@@ -258,28 +258,33 @@ __device__ inline R dot_vB(const V8<R>& w) {
     return acc;
 }
 
-// Whether the arithmetic of fd is exact on what the hydrodynamic solvers form
+// Whether the arithmetic of fd is exact on what the solvers form
 // from two primitive states: density and pressure in [2^-60, 2^60], velocities
 // zero or in [2^-100, 2^60].  Differences and averages of such values are zero
 // or at least 2^-210, wave speeds and their differences zero or at least
 // 2^-440, the numerators of the HLLC speeds zero or at least 2^-703 and their
 // quotients at most 2^900: every remainder a division or square root corrects
-// with is a normal number (>= 2^-969 before the correction).
+// with is a normal number (>= 2^-969 before the correction).  With a magnetic
+// field: density and pressure in [2^-30, 2^30], velocities and fields zero or in
+// [2^-100, 2^30]; hlld_wave checks what its longer chains make of them.
 template <int MASK>
 __device__ inline bool safe_states(const V8<double>& a, const V8<double>& b) {
     using V = VS<MASK>;
+    constexpr double HI = V::MHD ? 0x1p30 : 0x1p60, LO = V::MHD ? 0x1p-30 : 0x1p-60;
     double sum = (a.c[0] + b.c[0]) + (a.c[4] + b.c[4]);  // NaN and infinities fail the comparison
     int ex = 0;
 #pragma unroll
-    for (int i = 1; i < 4; ++i)
-        if (V::live(i)) {
+    for (int i = 1; i < 8; ++i)
+        if (V::live(i) && i != 4) {
             sum = sum + (ah_fabs(a.c[i]) + ah_fabs(b.c[i]));
             const int ea = __builtin_amdgcn_frexp_exp(a.c[i]), eb = __builtin_amdgcn_frexp_exp(b.c[i]);
             ex = min(ex, min(ea, eb));  // 0 for a zero
         }
     const double low = __builtin_fmin(__builtin_fmin(a.c[0], b.c[0]), __builtin_fmin(a.c[4], b.c[4]));
-    return sum <= 0x1p60 && low >= 0x1p-60 && ex >= -99;
+    return sum <= HI && low >= LO && ex >= -99;
 }
+// the same for a normal field
+__device__ inline bool safe_field(double Bn) { return ah_fabs(Bn) <= 0x1p30 && __builtin_amdgcn_frexp_exp(Bn) >= -99; }
 // the same for states derived from safe ones (averages, transverse corrections)
 template <class R>
 __device__ inline bool safe_derived(const V8<R>& a, const V8<R>& b) {
@@ -381,9 +386,11 @@ __device__ inline R spectral_radius(const V8<R>& w, R gamma) {
     const R a2 = gamma * p / rho;
     if constexpr (is_fd<R> && !V::MHD) return ah_fabs(u) + ah_sqrt(a2);  // finite, p > 0
     bool fin = true;
+    if constexpr (!is_fd<R>) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-        if (V::live(i)) fin = fin && ah_isfinite(w.c[i]);
+        for (int i = 0; i < 8; ++i)
+            if (V::live(i)) fin = fin && ah_isfinite(w.c[i]);
+    }
     R r;
     if constexpr (!V::MHD) {
         r = a2 >= R(0) ? ah_fabs(u) + ah_sqrt(a2) : ah_sqrt(ah_fabs(u * u - a2));
@@ -396,7 +403,8 @@ __device__ inline R spectral_radius(const V8<R>& w, R gamma) {
         const R cf2 = R(0.5) * (s + ah_sqrt(disc > R(0) ? disc : R(0)));
         r = ah_fabs(u) + ah_sqrt(cf2 > R(0) ? cf2 : R(0));
     }
-    return fin ? r : R(NAN);
+    if constexpr (is_fd<R>) return r;
+    else return fin ? r : R(NAN);
 }
 
 // ---- slope limiters (limiters.py:10-49); a backward, b forward difference ----
@@ -784,118 +792,189 @@ __device__ inline V8<double> flux_hllc_split(const Iface<double>& s, int sax, do
 // FP64 on the split path too: its region selection is discontinuous (both
 // Alfven speeds s_M - B_n / sqrt(rho*), the default F(w-)), and FP32 fast
 // speeds flipped a region of the Brio-Wu problem within six steps.
+// In two steps: the waves, from the interface states, then the flux, which takes
+// the conservative states and physical fluxes.  The side of the contact the
+// interface lies on is selected with the waves, so that only one side's energies
+// and differences are formed.
+template <class R>
+struct HlldWave {
+    R rs, mA, vA;             // the side's density; momentum (outer) and velocity (inner) along the axis
+    R m[2], v[2], B[2], Bi[2];  // the other two components: outer momentum, inner velocity, outer and inner field
+    R su, sSM, up, pM, sg, sp, vB;  // s - u, s - s_M, u (p + B^2/2), p* s_M, sqrt(rho*) sgn(Bn), wave speed, v.B
+    bool right, inner, star;  // the side; its inner state; a star state at all (solvers.py:226-231)
+};
+template <class R>
+__device__ inline HlldWave<double> wide(const HlldWave<R>& h) {
+    HlldWave<double> d;
+    d.rs = double(h.rs), d.mA = double(h.mA), d.vA = double(h.vA);
+    for (int i = 0; i < 2; ++i)
+        d.m[i] = double(h.m[i]), d.v[i] = double(h.v[i]), d.B[i] = double(h.B[i]), d.Bi[i] = double(h.Bi[i]);
+    d.su = double(h.su), d.sSM = double(h.sSM), d.up = double(h.up), d.pM = double(h.pM), d.sg = double(h.sg);
+    d.sp = double(h.sp), d.vB = double(h.vB);
+    d.right = h.right, d.inner = h.inner, d.star = h.star;
+    return d;
+}
+// In fd's arithmetic, on safe_states and a safe_field, ok says whether the bits
+// are the general ones.  From those ranges: fast speeds in [2^-31, 2^47], s - u
+// zero or in [2^-152, 2^49], the numerators of s_M and p* zero or in
+// [2^-416, 2^158].  With the checks that every divisor and rho* be at least
+// 2^-100 (dL, dR: 2^-150): s_M at most 2^212 and, as a multiple of 2^-466,
+// s_M - u zero or at least that; rho* at most 2^179, dL at most 2^292; so every
+// quotient so far is zero or in [2^-758, 2^363] and its remainder a multiple of
+// 2^-571.  The numerators of the inner states are checked themselves: zero or at
+// least 2^-800 (they cannot exceed 2^603).  Roots are taken of zero or at least
+// 2^-342, which the checks on the discriminants and rho* make non-negative.
+// Components that the state does not hold are zeros in every term, which fd
+// (all finite) leaves out.
+template <class R, int MASK>
+__device__ constexpr bool hlld_held(int i) { return !is_fd<R> || VS<MASK>::live(i); }
+template <class R, int MASK>
+__device__ inline R hlld_dot(const R* v, const R* B) {
+    R t = v[0] * B[0];
+    if (hlld_held<R, MASK>(6)) t = t + v[1] * B[1];
+    return hlld_held<R, MASK>(7) ? t + v[2] * B[2] : t;
+}
 template <class R, int MASK, int SAX>
-__device__ inline V8<R> flux_hlld(const Iface<R>& s, R Bn, R gamma) {
-    constexpr int A = SAX % 3, O = (SAX + 1) % 3, C = (SAX + 2) % 3;
-    auto cfast = [&](const V8<R>& w) {
+__device__ inline HlldWave<R> hlld_wave(const V8<R>& wL, const V8<R>& wR, R Bn, R gamma, bool* ok) {
+    constexpr int A = SAX % 3;
+    auto held = [](int i) { return hlld_held<R, MASK>(i); };
+    auto b2 = [&](const V8<R>& w) {
+        R t = w.c[5] * w.c[5];
+        if (held(6)) t = t + w.c[6] * w.c[6];
+        return held(7) ? t + w.c[7] * w.c[7] : t;
+    };
+    auto cfast = [&](const V8<R>& w, R nb, R& disc) {
         const R rho = w.c[0], p = w.c[4];
-        const R cs = ah_sqrt(gdiv(gamma * p, rho));
-        const R ca = gdiv(ah_sqrt((w.c[5] * w.c[5] + w.c[6] * w.c[6]) + w.c[7] * w.c[7]), ah_sqrt(rho));
-        const R cax = gdiv(w.c[5], ah_sqrt(rho));
+        const R cs = ah_sqrt(gdiv_pos(gamma * p, rho));
+        const R sr = ah_sqrt(rho);
+        const R ca = gdiv_pos(nb, sr);
+        const R cax = gdiv_pos(w.c[5], sr);
         const R cs2 = cs * cs, ca2 = ca * ca;
-        return ah_sqrt(R(0.5) * (cs2 + ca2 + ah_sqrt(sq(cs2 + ca2) - R(4) * cs2 * (cax * cax))));
+        disc = sq(cs2 + ca2) - R(4) * cs2 * (cax * cax);
+        return ah_sqrt(R(0.5) * (cs2 + ca2 + ah_sqrt(disc)));
     };
-    auto n2 = [](R a, R b, R c) {
-        R n = ah_sqrt((a * a + b * b) + c * c);
-        return n * n;
-    };
-    auto d3 = [](R a0, R b0, R a1, R b1, R a2, R b2) { return (a0 * b0 + a1 * b1) + a2 * b2; };
-    const V8<R>&wL = s.wm, &wR = s.wp, &QL = s.qm, &QR = s.qp;
     const R rhoL = wL.c[0], pL = wL.c[4], rhoR = wR.c[0], pR = wR.c[4];
     const R uL = wL.c[SAX + 1], uR = wR.c[SAX + 1];
-    const R cfL = cfast(wL), cfR = cfast(wR);
+    const R nbL = ah_sqrt(b2(wL)), nbR = ah_sqrt(b2(wR));  // fv.norm
+    R discL, discR;
+    const R cfL = cfast(wL, nbL, discL), cfR = cfast(wR, nbR, discR);
     const R umin = nmin(uL, uR), cmax = nmax(cfL, cfR);
     const R sL = umin - cmax, sR = umin + cmax;
-    const R bL2 = n2(wL.c[5], wL.c[6], wL.c[7]), bR2 = n2(wR.c[5], wR.c[6], wR.c[7]);
-    const R den = rhoL * (sL - uL) - rhoR * (sR - uR);
-    const R sM = gdiv(pR - pL + rhoL * uL * (sL - uL) - rhoR * uR * (sR - uR) + R(0.5) * bR2 - R(0.5) * bL2, den);
-    const R rLs = rhoL * gdiv(sL - uL, sL - sM), rRs = rhoR * gdiv(sR - uR, sR - sM);
-    const R sLs = sM - gdiv(wL.c[SAX + 5], ah_sqrt(rLs)), sRs = sM - gdiv(wR.c[SAX + 5], ah_sqrt(rRs));
-    const R ps = gdiv(rhoL * (pR + R(0.5) * bR2) * (sL - uL) - rhoR * (pL + R(0.5) * bL2) * (sR - uR) +
-                          rhoR * rhoL * (sL - uL) * (sR - uR),
-                      den);
-    const R Bn2 = Bn * Bn;
-    const R dL = rhoL * (sL - uL) * (sL - sM) - Bn2, dR = rhoR * (sR - uR) * (sR - sM) - Bn2;
-    const R vyLs = wL.c[O + 1] - Bn * wL.c[O + 5] * gdiv(sM - uL, dL);
-    const R vyRs = wR.c[O + 1] - Bn * wR.c[O + 5] * gdiv(sM - uR, dR);
-    const R vzLs = wL.c[C + 1] - Bn * wL.c[C + 5] * gdiv(sM - uL, dL);
-    const R vzRs = wR.c[C + 1] - Bn * wR.c[C + 5] * gdiv(sM - uR, dR);
-    const R ByLs = wL.c[O + 5] * gdiv(rhoL * sq(sL - uL) - Bn2, dL);
-    const R ByRs = wR.c[O + 5] * gdiv(rhoR * sq(sR - uR) - Bn2, dR);
-    const R BzLs = wL.c[C + 5] * gdiv(rhoL * sq(sL - uL) - Bn2, dL);
-    const R BzRs = wR.c[C + 5] * gdiv(rhoR * sq(sR - uR) - Bn2, dR);
-    V8<R> QLs, QRs;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) QLs.c[i] = QRs.c[i] = R(0);
-    QLs.c[0] = rLs;
-    QRs.c[0] = rRs;
-    QLs.c[A + 1] = rhoL * sM;
-    QRs.c[A + 1] = rhoR * sM;
-    QLs.c[O + 1] = rhoL * vyLs;
-    QRs.c[O + 1] = rhoR * vyRs;
-    QLs.c[C + 1] = rhoL * vzLs;
-    QRs.c[C + 1] = rhoR * vzRs;
-    QLs.c[A + 5] = QL.c[A + 5];
-    QRs.c[A + 5] = QR.c[A + 5];
-    QLs.c[O + 5] = ByLs;
-    QRs.c[O + 5] = ByRs;
-    QLs.c[C + 5] = BzLs;
-    QRs.c[C + 5] = BzRs;
-    const R vBL = d3(wL.c[1], wL.c[5], wL.c[2], wL.c[6], wL.c[3], wL.c[7]);
-    const R vBR = d3(wR.c[1], wR.c[5], wR.c[2], wR.c[6], wR.c[3], wR.c[7]);
-    const R mBLs = d3(QLs.c[1], QLs.c[5], QLs.c[2], QLs.c[6], QLs.c[3], QLs.c[7]);
-    const R mBRs = d3(QRs.c[1], QRs.c[5], QRs.c[2], QRs.c[6], QRs.c[3], QRs.c[7]);
-    QLs.c[4] = gdiv(QL.c[4] * (sL - uL) - uL * (pL + R(0.5) * bL2) + ps * sM + Bn * (vBL - mBLs), sL - sM);
-    QRs.c[4] = gdiv(QR.c[4] * (sR - uR) - uR * (pR + R(0.5) * bR2) + ps * sM + Bn * (vBR - mBRs), sR - sM);
-    const R sg = nsign(Bn);
+    const R bL2 = nbL * nbL, bR2 = nbR * nbR;
+    const R sLu = sL - uL, sRu = sR - uR;
+    const R den = rhoL * sLu - rhoR * sRu;
+    const R sM = gdiv_pos(pR - pL + rhoL * uL * sLu - rhoR * uR * sRu + R(0.5) * bR2 - R(0.5) * bL2, den);
+    const R sLM = sL - sM, sRM = sR - sM;
+    const R rLs = rhoL * gdiv_pos(sLu, sLM), rRs = rhoR * gdiv_pos(sRu, sRM);
     const R srL = ah_sqrt(rLs), srR = ah_sqrt(rRs), srs = srL + srR, srp = ah_sqrt(rRs * rLs);
-    const R vyss = gdiv(vyRs * srR + vyLs * srL + sg * (ByLs - ByRs), srs);
-    const R vzss = gdiv(vzRs * srR + vzLs * srL + sg * (BzLs - BzRs), srs);
-    const R Byss = gdiv(ByLs * srR + ByRs * srL + sg * (vyLs - vyRs) * srp, srs);
-    const R Bzss = gdiv(BzLs * srR + BzRs * srL + sg * (vzLs - vzRs) * srp, srs);
-    V8<R> QLss, QRss;
+    const R sLs = sM - gdiv_pos(wL.c[SAX + 5], srL), sRs = sM - gdiv_pos(wR.c[SAX + 5], srR);
+    const R ptL = pL + R(0.5) * bL2, ptR = pR + R(0.5) * bR2;
+    const R ps = gdiv_pos(rhoL * ptR * sLu - rhoR * ptL * sRu + rhoR * rhoL * sLu * sRu, den);
+    const R Bn2 = Bn * Bn;
+    const R dL = rhoL * sLu * sLM - Bn2, dR = rhoR * sRu * sRM - Bn2;
+    const R vqL = gdiv_pos(sM - uL, dL), vqR = gdiv_pos(sM - uR, dR);
+    const R BqL = gdiv_pos(rhoL * sq(sLu) - Bn2, dL), BqR = gdiv_pos(rhoR * sq(sRu) - Bn2, dR);
+    HlldWave<R> h;
+    // region select (solvers.py:226-231): regions 1 and 4 are the outer, 2 and 3
+    // the inner states, 0 F(w-) and 5 F(w+); later masks overwrite earlier ones
+    // (all evaluated: no branch parts the chains of solves side by side)
+    const bool r1 = (sL <= R(0)) & (R(0) < sLs), r2 = (sLs <= R(0)) & (R(0) < sM), r3 = (sM <= R(0)) & (R(0) < sRs),
+               r4 = (sRs <= R(0)) & (R(0) <= sR), r5 = sR < R(0);
+    const bool right = r3 | r4 | r5, inner = !(r4 | r5) & (r2 | r3);
+    h.right = right;
+    h.inner = inner;
+    h.star = !r5 & (r1 | r2 | r3 | r4);
+    auto pick = [&](R l, R r) { return right ? r : l; };
+    const R sg = nsign(Bn), rho = pick(rhoL, rhoR);
+    h.rs = pick(rLs, rRs);
+    h.mA = rho * sM;
+    h.vA = sM;
+    int ex = 0;  // least exponent of the inner states' numerators
 #pragma unroll
-    for (int i = 0; i < 8; ++i) QLss.c[i] = QRss.c[i] = R(0);
-    QLss.c[0] = rLs;
-    QRss.c[0] = rRs;
-    QLss.c[A + 1] = sM;
-    QRss.c[A + 1] = sM;
-    QLss.c[O + 1] = vyss;
-    QRss.c[O + 1] = vyss;
-    QLss.c[C + 1] = vzss;
-    QRss.c[C + 1] = vzss;
-    QLss.c[A + 5] = QLs.c[A + 5];
-    QRss.c[A + 5] = QRs.c[A + 5];
-    QLss.c[O + 5] = Byss;
-    QRss.c[O + 5] = Byss;
-    QLss.c[C + 5] = Bzss;
-    QRss.c[C + 5] = Bzss;
-    const R mBLss = d3(QLss.c[1], QLss.c[5], QLss.c[2], QLss.c[6], QLss.c[3], QLss.c[7]);
-    const R mBRss = d3(QRss.c[1], QRss.c[5], QRss.c[2], QRss.c[6], QRss.c[3], QRss.c[7]);
-    QLss.c[4] = QLs.c[4] - srL * sg * (mBLs - mBLss);
-    QRss.c[4] = QRs.c[4] - srR * sg * (mBRs - mBRss);
-    // region select (solvers.py:226-231), later masks overwrite earlier ones
-    int reg = 0;  // 0: F(w-)
-    if ((sL <= R(0)) && (R(0) < sLs)) reg = 1;
-    if ((sLs <= R(0)) && (R(0) < sM)) reg = 2;
-    if ((sM <= R(0)) && (R(0) < sRs)) reg = 3;
-    if ((sRs <= R(0)) && (R(0) <= sR)) reg = 4;
-    if (sR < R(0)) reg = 5;
-    V8<R> F;
+    for (int m = 0; m < 2; ++m) {
+        const int i = (A + 1 + m) % 3;
+        if (!held(i + 5)) {
+            h.m[m] = h.v[m] = h.B[m] = h.Bi[m] = R(0);
+            continue;
+        }
+        const R vL = wL.c[i + 1] - Bn * wL.c[i + 5] * vqL, vR = wR.c[i + 1] - Bn * wR.c[i + 5] * vqR;
+        const R BL = wL.c[i + 5] * BqL, BR = wR.c[i + 5] * BqR;
+        const R nv = vR * srR + vL * srL + sg * (BL - BR), nB = BL * srR + BR * srL + sg * (vL - vR) * srp;
+        h.m[m] = rho * pick(vL, vR);
+        h.B[m] = pick(BL, BR);
+        h.v[m] = gdiv_pos(nv, srs);
+        h.Bi[m] = gdiv_pos(nB, srs);
+        if constexpr (is_fd<R>)
+            ex = min(ex, min(__builtin_amdgcn_frexp_exp(nv.v), __builtin_amdgcn_frexp_exp(nB.v)));
+    }
+    h.su = pick(sLu, sRu);
+    h.sSM = pick(sLM, sRM);
+    h.up = pick(uL, uR) * pick(ptL, ptR);
+    h.pM = ps * sM;
+    h.sg = pick(srL, srR) * sg;
+    h.sp = inner ? pick(sLs, sRs) : pick(sL, sR);
+    R v[3], B[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        v[i] = pick(wL.c[i + 1], wR.c[i + 1]);
+        B[i] = pick(wL.c[i + 5], wR.c[i + 5]);
+    }
+    h.vB = hlld_dot<R, MASK>(v, B);
+    if constexpr (is_fd<R>) {
+        const double d1 = imin(imin_abs(den.v, sLM.v), imin(imin(rLs.v, rRs.v), ah_fabs(sRM.v)));
+        *ok = (d1 >= 0x1p-100) & (imin_abs(dL.v, dR.v) >= 0x1p-150) & (imin(discL.v, discR.v) >= 0.0) & (ex >= -799);
+    }
+    return h;
+}
+template <class R, int MASK, int SAX>
+__device__ inline V8<R> hlld_flux(const HlldWave<R>& h, R Bn, const V8<R>& QL, const V8<R>& QR, const V8<R>& fL,
+                                  const V8<R>& fR) {
+    constexpr int A = SAX % 3, O = (SAX + 1) % 3, C = (SAX + 2) % 3;
+    const bool right = h.right, inner = h.inner, star = h.star;
+    V8<R> Q, Fb;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        R v;
-        switch (reg) {
-            case 1: v = s.fm.c[i] + (QLs.c[i] - QL.c[i]) * sL; break;
-            case 2: v = s.fm.c[i] + (QLss.c[i] - QLs.c[i]) * sLs; break;
-            case 3: v = s.fp.c[i] + (QRss.c[i] - QRs.c[i]) * sRs; break;
-            case 4: v = s.fp.c[i] + (QRs.c[i] - QR.c[i]) * sR; break;
-            case 5: v = s.fp.c[i]; break;
-            default: v = s.fm.c[i]; break;
-        }
-        F.c[i] = v;
+        Q.c[i] = right ? QR.c[i] : QL.c[i];
+        Fb.c[i] = right ? fR.c[i] : fL.c[i];
+    }
+    R ms[3], vi[3], Bs[3], Bi[3];  // by component
+    ms[A] = h.mA, ms[O] = h.m[0], ms[C] = h.m[1];
+    vi[A] = h.vA, vi[O] = h.v[0], vi[C] = h.v[1];
+    Bs[A] = Bi[A] = Q.c[A + 5];
+    Bs[O] = h.B[0], Bs[C] = h.B[1];
+    Bi[O] = h.Bi[0], Bi[C] = h.Bi[1];
+    const R mBs = hlld_dot<R, MASK>(ms, Bs), mBi = hlld_dot<R, MASK>(vi, Bi);
+    const R Es = gdiv(Q.c[4] * h.su - h.up + h.pM + Bn * (h.vB - mBs), h.sSM);
+    const R Ei = Es - h.sg * (mBs - mBi);
+    auto out = [&](int i, R qs, R qi) {
+        const R d = (inner ? qi - qs : qs - Q.c[i]) * h.sp;
+        return star ? Fb.c[i] + d : Fb.c[i];
+    };
+    V8<R> F;
+    F.c[0] = out(0, h.rs, h.rs);
+    F.c[4] = out(4, Es, Ei);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        F.c[i + 1] = out(i + 1, ms[i], vi[i]);
+        F.c[i + 5] = out(i + 5, Bs[i], Bi[i]);
     }
     return F;
+}
+// waves and flux; fd's flux divides by the general division
+template <class R, int MASK, int SAX>
+__device__ inline V8<R> flux_hlld(const Iface<R>& s, R Bn, R gamma, bool* ok) {
+    const HlldWave<R> h = hlld_wave<R, MASK, SAX>(s.wm, s.wp, Bn, gamma, ok);
+    if constexpr (is_fd<R>) {
+        auto d = [](const V8<R>& v) {
+            V8<double> r;
+            for (int i = 0; i < 8; ++i) r.c[i] = v.c[i].v;
+            return r;
+        };
+        const V8<double> F = hlld_flux<double, MASK, SAX>(wide(h), Bn.v, d(s.qm), d(s.qp), d(s.fm), d(s.fp));
+        V8<R> r;
+        for (int i = 0; i < 8; ++i) r.c[i] = R(F.c[i]);
+        return r;
+    } else return hlld_flux<R, MASK, SAX>(h, Bn, s.qm, s.qp, s.fm, s.fp);
 }
 
 // ---- Osher-Solomon flux with the Dumbser-Toro path integral (solvers.py:236-284)

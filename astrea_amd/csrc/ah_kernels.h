@@ -473,9 +473,10 @@ __device__ inline V8<double> jac_state(const V8<double>& wp, const V8<double>& w
     }
 }
 
+// ok (HLLD in fd's arithmetic): whether the result's bits are the general ones
 template <class R, int MASK, int SOLVER, int AX>
 __device__ inline V8<R> riemann(const Iface<R>& s, R lam, int sax, R Bn, R gamma, int mom, bool physical,
-                               bool split = false) {
+                               bool split = false, bool* ok = nullptr) {
     if constexpr (SOLVER == LLF || SOLVER == LW)
         return flux_llf<R, MASK>(s, lam);
     else if constexpr (SOLVER == HLLC)
@@ -488,7 +489,7 @@ __device__ inline V8<R> riemann(const Iface<R>& s, R lam, int sax, R Bn, R gamma
     else if constexpr (SOLVER == ES)
         return flux_es<MASK>(s, sax, gamma);
     else
-        return sax == 0 ? flux_hlld<R, MASK, 0>(s, Bn, gamma) : flux_hlld<R, MASK, 1>(s, Bn, gamma);
+        return sax == 0 ? flux_hlld<R, MASK, 0>(s, Bn, gamma, ok) : flux_hlld<R, MASK, 1>(s, Bn, gamma, ok);
 }
 
 // Osher-Solomon: a non-finite flux marks the step failed (flux_dots returns
@@ -563,8 +564,8 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
     constexpr bool HO = (RECON == PPM || RECON >= WENO3);
     // interface states in fd's range are solved in its arithmetic (wave-uniform
     // choice): 192 ragged PPM/HLLC problems 1.81 -> 1.76 ms per 16 steps
-    constexpr bool FAST = std::is_same<R, double>::value && !SPLIT && !V::MHD && RECON != PCM &&
-                          (SOLVER == LLF || SOLVER == HLLC);
+    constexpr bool FAST = std::is_same<R, double>::value && !SPLIT && RECON != PCM &&
+                          (V::MHD ? SOLVER == HLLD : (SOLVER == LLF || SOLVER == HLLC));
     constexpr int HW_L = 5, HW_R = 6;                 // wS window [s0-5, s0+TS+6)
     constexpr int NQ = TS + HW_L + HW_R + 2;           // q window [s0-6, s0+TS+7)
     constexpr int NW = TS + HW_L + HW_R;
@@ -854,6 +855,8 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
         R Bn = R(0);
         if constexpr (SOLVER == HLLD) Bn = W(e(k)).c[5];
         V8<R> F;
+        R rk = R(0);
+        bool ok = true;
         // conversions, fluxes and solve in arithmetic A
         auto solve = [&](auto arith) {
             using A = decltype(arith);
@@ -875,17 +878,21 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
                 g.fp = phys_flux<A, MASK, 0>(g.wp, A(gR));
             }
             if constexpr (MERGED) {
-                if constexpr (SPLIT) own_radius(k, radius<MASK, 0, true>(jac_state<MASK, true, RECON != PLM>(f.wp, f.wm), gamma));
-                else own_radius(k, radius_of(arith, f.wp, f.wm));
+                if constexpr (SPLIT) rk = radius<MASK, 0, true>(jac_state<MASK, true, RECON != PLM>(f.wp, f.wm), gamma);
+                else rk = radius_of(arith, f.wp, f.wm);
             }
-            F = cast8<R, A, MASK>(riemann<A, MASK, SOLVER, 0>(g, A(lam), sax, A(Bn), A(gR), 1, a.compat != 0, SPLIT));
+            F = cast8<R, A, MASK>(riemann<A, MASK, SOLVER, 0>(g, A(lam), sax, A(Bn), A(gR), 1, a.compat != 0, SPLIT, &ok));
         };
         if constexpr (FAST) {
-            if (__all(safe_states<MASK>(f.wm, f.wp))) solve(fd(0.0));
-            else solve(R(0));
+            ok = safe_states<MASK>(f.wm, f.wp);
+            if constexpr (V::MHD) ok = ok && safe_field(Bn);
+            const bool fast = __all(ok);
+            if (fast) solve(fd(0.0));
+            if (!fast || (V::MHD && !__all(ok))) solve(R(0));
         } else {
             solve(R(0));
         }
+        if constexpr (MERGED) own_radius(k, rk);
         dots_fail<SOLVER, MASK>(F, ps);
         if constexpr (RECON == PPM) {
             if (a.av) {

@@ -17,10 +17,13 @@
 // issue, a line costing 2.0e7 / (1024^2 / 63) wave instructions where the tiles
 // spend 4.2e7.  Per launch (x, y sweep) at 1024^2 PPM/HLLC, tiles -> marching:
 // 110, 119 -> 62, 69 us; at 2048^2 PLM/HLLC 307, 390 -> 200, 216 us; at 768^2
-// WENO5/HLLD 135, 149 -> 104, 102 us.  Measured and left out: reading the
+// WENO5/HLLD 141, 153 -> 98, 94 us (113, 108 with general divisions and
+// roots; with one wave on a SIMD, the waves of a line's two solves run side by
+// side).  Measured and left out: reading the
 // states a whole line ahead (the registers spill, and a spill's reload waits
 // for the loads before it), one wave per SIMD with all in registers (33 us of
-// issue in 70), the line's values in LDS too, and two lines per loop turn.
+// issue in 70), the line's values in LDS too, two lines per loop turn, and for
+// MHD the next line's states a whole line ahead (100, 104 us).
 #pragma once
 #include "ah_kernels.h"
 
@@ -78,9 +81,10 @@ template <int MASK, int SOLVER, int CONV, int AX>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves<MASK>())))
 void flux2d_march_kernel(SweepArgs a) {
     using V = VS<MASK>;
+    using Wave = typename std::conditional<SOLVER == HLLD, HlldWave<double>, HllcWave<double>>::type;
     constexpr int NV = V::NV;
     constexpr bool LAM = SOLVER == LLF;
-    constexpr bool FAST = !V::MHD;
+    constexpr bool FAST = !V::MHD || SOLVER == HLLD;
     static_assert(CONV == 1 || CONV == 2, "the cell-centred form reads the stage input: flux2d_kernel");
     // x sweep: the lanes lie across the state's rows, so four lines of flux
     // differences are turned in LDS and written as 32-byte segments
@@ -159,7 +163,7 @@ void flux2d_march_kernel(SweepArgs a) {
     }
     MarchLine<MASK> x;      // face-averaged quantities of the line before
     V8<double> cwm, cwp;    // corrected interface states of the line before
-    HllcWave<double> wavx;  // HLLC: the waves of its second solve in their place
+    Wave wavx;              // HLLC, HLLD: the waves of its second solve in their place
     double lamx = 0.0, bnx = 0.0, lmax = 0.0;
     bool bad = false;
     if constexpr (FAST) okw = __all(safe_states<MASK>(wm, wp));
@@ -167,7 +171,7 @@ void flux2d_march_kernel(SweepArgs a) {
     for (int c = c0; c <= t1; ++c) {
         MarchLine<MASK> y;
         V8<double> ywm, ywp;
-        HllcWave<double> wavy;
+        Wave wavy;
         double lamy = 0.0, bny = 0.0;
         const bool past = edge && c == nt;  // beyond the edge: the line before again
         if (!past) {
@@ -179,6 +183,9 @@ void flux2d_march_kernel(SweepArgs a) {
             ywp = corr8<MASK>(wp, fwp, dwp);
             const bool town = c >= t0 && c < t1;
             double em_n, ep_n;
+            V8<double> gm, gp;  // the differences of the conservative states to the next line
+            bool ok = true;
+            double ro = 0.0;
             // the first solve of line c in arithmetic R
             auto first = [&](auto tag) {
                 using R = decltype(tag);
@@ -198,11 +205,10 @@ void flux2d_march_kernel(SweepArgs a) {
 #pragma unroll
                     for (int i = 0; i < 8; ++i)
                         if (V::live(i)) {
-                            const double gm = double(hpm.c[i]) - qcm.c[i], gp = double(hpp.c[i]) - qcp.c[i];
-                            s.qm.c[i] = s.qm.c[i] + R(K24 * (gm - dpm.c[i]));
-                            s.qp.c[i] = s.qp.c[i] + R(K24 * (gp - dpp.c[i]));
-                            dpm.c[i] = gm;
-                            dpp.c[i] = gp;
+                            gm.c[i] = double(hpm.c[i]) - qcm.c[i];
+                            gp.c[i] = double(hpp.c[i]) - qcp.c[i];
+                            s.qm.c[i] = s.qm.c[i] + R(K24 * (gm.c[i] - dpm.c[i]));
+                            s.qp.c[i] = s.qp.c[i] + R(K24 * (gp.c[i] - dpp.c[i]));
                         }
                 }
                 em_n = double(hpm.c[4]);
@@ -216,9 +222,7 @@ void flux2d_march_kernel(SweepArgs a) {
                     // the chains that the block runs side by side
                     const V8<R> st = CONV == 1 ? arith_avg<R, MASK>(s.wp, s.wm) : roe_avg<R, MASK>(s.wp, s.wm);
                     double r = double(spectral_radius<R, MASK, AX>(st, gR));
-                    const double ro = (town & jown) ? r : 0.0;
-                    bad = bad | !(ro <= 1.7976931348623157e308);
-                    lmax = ((ro > lmax) | (ro != ro)) ? ro : lmax;
+                    ro = (town & jown) ? r : 0.0;
                     if constexpr (LAM) {
                         double rn = lane_next(r);
                         if (edge) {
@@ -241,6 +245,19 @@ void flux2d_march_kernel(SweepArgs a) {
                     wavy.mom = double(h2.mom);
                     wavy.en = double(h2.en);
                     wavy.sel = h2.sel;
+                } else if constexpr (SOLVER == HLLD) {
+                    auto both = [&](auto axis) {
+                        constexpr int S = decltype(axis)::value;
+                        bool ok2 = true;
+                        const HlldWave<R> h1 = hlld_wave<R, MASK, S>(s.wm, s.wp, R(bny), gR, &ok);
+                        const HlldWave<R> h2 = hlld_wave<R, MASK, S>(up(ywm), up(ywp), R(bny), gR, &ok2);
+                        ok = ok && ok2;
+                        auto dn = [](const V8<R>& v) { return cast8<double, R, MASK>(v); };
+                        F = cast8<R, double, MASK>(hlld_flux<double, MASK, S>(wide(h1), bny, dn(s.qm), dn(s.qp), dn(s.fm), dn(s.fp)));
+                        wavy = wide(h2);
+                    };
+                    if (sax == 0) both(std::integral_constant<int, 0>{});
+                    else both(std::integral_constant<int, 1>{});
                 } else {
                     F = riemann<R, MASK, SOLVER, AX>(s, R(lamy), sax, R(bny), gR, sax + 1, a.compat != 0);
                 }
@@ -253,12 +270,23 @@ void flux2d_march_kernel(SweepArgs a) {
             bool fast = false;
             if constexpr (FAST) {
                 const bool okh = __all(safe_states<MASK>(hm, hp));
-                fast = okl && okw && okh && __all(safe_derived(ywm, ywp));
+                fast = okl && okw && okh;
+                if constexpr (V::MHD) fast = fast && __all(safe_states<MASK>(ywm, ywp) && safe_field(bny));
+                else fast = fast && __all(safe_derived(ywm, ywp));
                 okl = okw;
                 okw = okh;
             }
-            if (FAST && fast) first(fd(0.0));
-            else first(0.0);
+            if (FAST && fast) {
+                first(fd(0.0));
+                if constexpr (V::MHD) fast = __all(ok);
+            }
+            if (!(FAST && fast)) first(0.0);
+            bad = bad | !(ro <= 1.7976931348623157e308);
+            lmax = ((ro > lmax) | (ro != ro)) ? ro : lmax;
+            if constexpr (CONV == 2) {
+                dpm = gm;
+                dpp = gp;
+            }
             em_ = em_n;
             ep_ = ep_n;
             wm = hm;
@@ -317,6 +345,9 @@ void flux2d_march_kernel(SweepArgs a) {
                 V8<double> F;
                 if constexpr (SOLVER == HLLC)
                     F = hllc_flux<double, MASK>(wavx, s.qm, s.qp, s.fm, s.fp, mom, a.compat != 0);
+                else if constexpr (SOLVER == HLLD)
+                    F = sax == 0 ? hlld_flux<double, MASK, 0>(wavx, bnx, s.qm, s.qp, s.fm, s.fp)
+                                 : hlld_flux<double, MASK, 1>(wavx, bnx, s.qm, s.qp, s.fm, s.fp);
                 else F = riemann<double, MASK, SOLVER, AX>(s, lamx, sax, bnx, gamma, sax + 1, a.compat != 0);
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
