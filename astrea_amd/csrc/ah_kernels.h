@@ -177,6 +177,43 @@ __device__ inline R flat_chi_at(const Acc& W, int flattener, int mm) {
     return flat_chi<R>(flattener, p2.c[4], p1.c[4], q1.c[4], q2.c[4], p1.c[AX + 1], q1.c[AX + 1]);
 }
 
+// WENO of one cell, every component, in arithmetic A.  Two thirds of the issue
+// of its launch is the weights' divisions: fd takes WENO5 at 768^2 MHD from
+// 62/61 to 55/53 us per launch (x/y), at 517 x 333 from 15.0/16.6 to 13.5/14.4.
+template <class A, class R, int MASK, int RECON, class Acc>
+__device__ inline void weno_cell(const Acc& W, int ce, V8<R>& wL, V8<R>& wR) {
+    constexpr int H = RECON == WENO3 ? 1 : (RECON == WENO5 ? 2 : 3);
+    V8<R> w[2 * H + 1];
+#pragma unroll
+    for (int k = 0; k < 2 * H + 1; ++k) w[k] = W(ce - H + k);
+    wL = wR = zero8<R, MASK>();
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        if (!VS<MASK>::live(c)) continue;
+        A l, r;
+        auto x = [&](int k) { return A(w[k].c[c]); };
+        if constexpr (RECON == WENO3) weno3<A>(x(0), x(1), x(2), l, r);
+        else if constexpr (RECON == WENO5) weno5<A>(x(0), x(1), x(2), x(3), x(4), l, r);
+        else weno7<A>(x(0), x(1), x(2), x(3), x(4), x(5), x(6), l, r);
+        wL.c[c] = R(l);
+        wR.c[c] = R(r);
+    }
+}
+
+// Whether fd's divisions are exact in the WENO weights of states of such a size:
+// the smoothness indicators' squares lie in [1e-12, 2^255] (fifth and third
+// order, sums of squares, up to 2^60; the seventh order's expanded forms stay
+// within 1e-6 / 4 of theirs up to 2^6), so weights, sums and ratios in
+// [2^-300, 2^42].
+template <int MASK, int RECON, class R>
+__device__ inline bool safe_weno(const V8<R>& w) {
+    double sum = 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if (VS<MASK>::live(i)) sum = sum + ah_fabs(double(w.c[i]));  // NaN fails the comparison
+    return sum <= (RECON == WENO7 ? 0x1p6 : 0x1p60);
+}
+
 // One cell's reconstruction from a window accessor W(m) that returns the
 // primitive state at sweep position m (already boundary mapped).  `ce` is the
 // evaluation position of the cell; chi_at(mm) returns flat_chi_at(W, mm)
@@ -248,21 +285,7 @@ __device__ inline void recon_cell(const Acc& W, int ce, int limiter, int flatten
                         d3p2, wL.c[c], wR.c[c]);
         }
     } else {
-        constexpr int H = RECON == WENO3 ? 1 : (RECON == WENO5 ? 2 : 3);
-        V8<R> w[7];
-#pragma unroll
-        for (int k = 0; k < 2 * H + 1; ++k) w[k] = W(ce - H + k);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            if (!V::live(c)) continue;
-            if constexpr (RECON == WENO3)
-                weno3<R>(w[0].c[c], w[1].c[c], w[2].c[c], wL.c[c], wR.c[c]);
-            else if constexpr (RECON == WENO5)
-                weno5<R>(w[0].c[c], w[1].c[c], w[2].c[c], w[3].c[c], w[4].c[c], wL.c[c], wR.c[c]);
-            else
-                weno7<R>(w[0].c[c], w[1].c[c], w[2].c[c], w[3].c[c], w[4].c[c], w[5].c[c], w[6].c[c], wL.c[c],
-                         wR.c[c]);
-        }
+        weno_cell<R, R, MASK, RECON>(W, ce, wL, wR);
     }
 }
 
@@ -634,6 +657,9 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
     }
     __syncthreads();
     // B: primitive cell averages wS on the window (FP64, then cast)
+    // WENO weights in fd's arithmetic if all of the window lies in its range
+    constexpr bool WENO_FD = RECON >= WENO3 && std::is_same<R, double>::value;
+    bool wok = true;
     for (int i = threadIdx.x; i < NW; i += blockDim.x) {
         const int iq = e(bw + i) - bq;
         V8<double> w;
@@ -665,8 +691,10 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
 #pragma unroll
         for (int c = 0; c < 8; ++c)
             if (V::live(c)) ws[V::slot(c)][i] = R(w.c[c]);
+        if constexpr (WENO_FD) wok = wok & safe_weno<MASK, RECON>(w);
     }
-    __syncthreads();
+    if constexpr (WENO_FD) wok = __syncthreads_and(wok);
+    else __syncthreads();
     struct WAcc {
         R (*ws)[NW];
         int bw, N, bc;
@@ -751,6 +779,8 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
                 else if constexpr (RECON == PPM)
                     recon_cell<R, MASK, RECON, 0>(Wc, Wc.e(bcl + i), a.limiter, a.flattener, L, Rr,
                                                   [&](int mm) { return chi_s[mm - (s0 - 3)]; });
+                else if (WENO_FD && wok)
+                    weno_cell<typename std::conditional<WENO_FD, fd, R>::type, R, MASK, RECON>(Wc, Wc.e(bcl + i), L, Rr);
                 else
                     recon_cell<R, MASK, RECON, 0>(Wc, Wc.e(bcl + i), a.limiter, a.flattener, L, Rr);
 #pragma unroll
@@ -1077,6 +1107,9 @@ void recon2d_kernel(SweepArgs a) {
     }
     __syncthreads();
     // B: wS for s in [s0-4, s0+TS+4), own rows t in [t0, t0+TT)
+    // WENO weights in fd's arithmetic if all of the window lies in its range
+    constexpr bool WENO_FD = RECON >= WENO3 && std::is_same<R, double>::value;
+    bool wok = true;
     for (int i = threadIdx.x; i < TT * NWS; i += blockDim.x) {
         const int it = i / NWS, is = i % NWS;
         const int t = t0 + it;
@@ -1107,8 +1140,10 @@ void recon2d_kernel(SweepArgs a) {
 #pragma unroll
         for (int c = 0; c < 8; ++c)
             if (V::live(c)) ws[V::slot(c)][it][is] = R(w.c[c]);
+        if constexpr (WENO_FD) wok = wok & safe_weno<MASK, RECON>(w);
     }
-    __syncthreads();
+    if constexpr (WENO_FD) wok = __syncthreads_and(wok);
+    else __syncthreads();
     // C: reconstruct own cells, write wL/wR (sweep frame [t][s])
     R* wLo = reinterpret_cast<R*>(a.wL);
     R* wRo = reinterpret_cast<R*>(a.wR);
@@ -1185,6 +1220,8 @@ void recon2d_kernel(SweepArgs a) {
         if constexpr (TWO)
             ppm_shared_cell<R, MASK>(W, s, s0 - 2, s0 - 1, [&](int v, int j) { return d2_s[v][it][j]; },
                                      [&](int v, int j) { return fc_s[v][it][j]; }, L, Rr);
+        else if (WENO_FD && wok)
+            weno_cell<typename std::conditional<WENO_FD, fd, R>::type, R, MASK, RECON>(W, s, L, Rr);
         else
             recon_cell<R, MASK, RECON, AX>(W, s, a.limiter, a.flattener, L, Rr);
         const long long o = fo + (long long)t * ns + s;

@@ -231,3 +231,24 @@ def test_short_divisions_and_roots_of_hlld_give_the_general_bits(shape, subgrid,
                     # strong shocks have roots of negative densities, and NaNs, in both
                     assert np.array_equal(got[q][ax]["flux"][..., i], want[..., i], equal_nan=True), (c, q, ax, i)
                 assert got[q][ax]["eigmax"] == np.ldexp(ref[q][ax]["eigmax"], c)
+
+
+@pytest.mark.parametrize("shape", [(30,), (243,), (33, 9), (70, 40)], ids=str)
+@pytest.mark.parametrize("subgrid", ["weno3", "weno5", "weno7"])
+def test_short_divisions_of_the_weno_weights_give_the_general_bits(shape, subgrid):
+    """One cell of huge velocity takes its
+    tile's weights to the general arithmetic; the interfaces whose stencils do
+    not reach it keep their bits."""
+    base = _grid(shape, 41)
+    far = base.copy()
+    at = tuple(n // 2 for n in shape)
+    rho = far[at][0]
+    far[at][1] = rho * 2.0 ** (70 if subgrid != "weno7" else 9)
+    far[at][4] += .5 * far[at][1] ** 2 / rho
+    ref, got = _fluxes(base, subgrid, "hllc", "edge"), _fluxes(far, subgrid, "hllc", "edge")
+    for ax in range(len(shape)):
+        f, g = (x[0][ax]["flux"].reshape(shape[ax] + 1, -1, 8) for x in (ref, got))
+        keep = np.abs(np.arange(len(f)) - at[ax] - .5) > 8  # conversion, stencil and interface reach less
+        for t in range(f.shape[1]):
+            sel = keep if len(shape) == 1 or abs(t - at[1 - ax]) <= 8 else np.ones_like(keep)
+            assert np.array_equal(f[sel, t], g[sel, t]), (ax, t)
