@@ -61,10 +61,10 @@ inline void set2d(KernelSet* ks) {
         ks->tts = TTS;
         ks->ttt = TTT;
         ks->trecon[0] = [](const MhdArgs& a, int nb, hipStream_t s) {
-            if (nb > 0) hipLaunchKernelGGL((trecon_kernel<R, MASK, 0, TTS, TTT>), dim3(nb), dim3(256), 0, s, a);
+            if (nb > 0) hipLaunchKernelGGL((trecon_kernel<R, MASK, 0, TTS, TTT>), dim3(nb), dim3(64 * VS<MASK>::NV), 0, s, a);
         };
         ks->trecon[1] = [](const MhdArgs& a, int nb, hipStream_t s) {
-            if (nb > 0) hipLaunchKernelGGL((trecon_kernel<R, MASK, 1, TTS, TTT>), dim3(nb), dim3(256), 0, s, a);
+            if (nb > 0) hipLaunchKernelGGL((trecon_kernel<R, MASK, 1, TTS, TTT>), dim3(nb), dim3(64 * VS<MASK>::NV), 0, s, a);
         };
         ks->corner = [](const MhdArgs& a, int nb, hipStream_t s) {
             if (nb > 0) hipLaunchKernelGGL((corner_kernel<R, MASK, TTS, TTT>), dim3(nb), dim3(256), 0, s, a);
