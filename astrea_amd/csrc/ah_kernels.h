@@ -1220,6 +1220,9 @@ void recon2d_kernel(SweepArgs a) {
         if constexpr (TWO)
             ppm_shared_cell<R, MASK>(W, s, s0 - 2, s0 - 1, [&](int v, int j) { return d2_s[v][it][j]; },
                                      [&](int v, int j) { return fc_s[v][it][j]; }, L, Rr);
+        else if constexpr (RECON == PPM)
+            recon_cell<R, MASK, RECON, AX>(W, s, a.limiter, a.flattener, L, Rr,
+                                           [&](int mm) { return chi_s[it][mm - (s0 - 2)]; });
         else if (WENO_FD && wok)
             weno_cell<typename std::conditional<WENO_FD, fd, R>::type, R, MASK, RECON>(W, s, L, Rr);
         else
