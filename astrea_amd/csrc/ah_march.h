@@ -356,7 +356,9 @@ void flux2d_march_kernel(SweepArgs a) {
                         F.c[i] = F.c[i] - K24 * (d - dback[4][V::slot(i)][lane]);
                         dback[4][V::slot(i)][lane] = d;
                     }
-                if (a.flux_out && k <= ns && (own || k == ns)) {
+                // (the interface behind the last cell is the last tile's: a tile
+                // before it may reach it too, with a lane that has no neighbour)
+                if (a.flux_out && (own || (lane == width && k == ns))) {
 #pragma unroll
                     for (int i = 0; i < 8; ++i)
                         if (V::live(i)) a.flux_out[V::slot(i) * a.flux_plane + (long long)k * nt + t] = F.c[i];

@@ -287,3 +287,24 @@ def test_corner_reconstruction_around_its_tiles(shape, boundary):
     out = out.cpu().numpy() if hasattr(out, "cpu") else np.asarray(out)
     for i in range(8):
         assert np.abs(out[..., i] - ref[..., i]).max() <= 1e-13 * max(np.abs(ref[..., i]).max(), 1.), i
+
+
+@pytest.mark.parametrize("shape", [(4000, 63), (63, 4000)], ids=str)
+@pytest.mark.parametrize("subgrid", ["plm", "ppm"])
+def test_marching_llf_writes_the_last_interface_from_the_last_tile(shape, subgrid):
+    """A side of 63 cells splits into tiles of 31 and 32: the first one's last
+    lane reaches interface 63, which only the second may write (periodic: the
+    first has not the neighbour's radius there)."""
+    import torch
+    from astrea_amd.plan import Plan
+    from tests.test_zz_no_alloc import _static_call
+    plan = Plan(2, subgrid, "llf", "ssprk(3,3)",
+                [dict(n0=shape[0], n1=shape[1], boundary="wrap", dx=1 / 512, gamma=1.4, cfl=.4, t_end=1e9)], varmask=0x17)
+    plan.load([torch.from_numpy(_grid(shape, 5)).cuda()])
+    for parity in (0, 1):
+        ref = plan.evolve_space(parity)
+        rc, f0, f1, eig = _static_call(plan, parity)
+        assert rc == 0
+        assert torch.equal(f0, ref[0]["raw"]) and torch.equal(f1, ref[1]["raw"])
+        assert eig == [ref[0]["eigmax"], ref[1]["eigmax"]]
+    plan.close()
