@@ -177,7 +177,7 @@ __device__ inline R flat_chi_at(const Acc& W, int flattener, int mm) {
     return flat_chi<R>(flattener, p2.c[4], p1.c[4], q1.c[4], q2.c[4], p1.c[AX + 1], q1.c[AX + 1]);
 }
 
-// WENO of one cell, every component, in arithmetic A.  Two thirds of the issue
+// WENO of one cell, every component, in arithmetic fd.  Two thirds of the issue
 // of its launch is the weights' divisions: fd takes WENO5 at 768^2 MHD from
 // 62/61 to 55/53 us per launch (x/y), at 517 x 333 from 15.0/16.6 to 13.5/14.4.
 template <class A, class R, int MASK, int RECON, class Acc>
@@ -285,7 +285,21 @@ __device__ inline void recon_cell(const Acc& W, int ce, int limiter, int flatten
                         d3p2, wL.c[c], wR.c[c]);
         }
     } else {
-        weno_cell<R, R, MASK, RECON>(W, ce, wL, wR);
+        constexpr int H = RECON == WENO3 ? 1 : (RECON == WENO5 ? 2 : 3);
+        V8<R> w[7];
+#pragma unroll
+        for (int k = 0; k < 2 * H + 1; ++k) w[k] = W(ce - H + k);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            if (!V::live(c)) continue;
+            if constexpr (RECON == WENO3)
+                weno3<R>(w[0].c[c], w[1].c[c], w[2].c[c], wL.c[c], wR.c[c]);
+            else if constexpr (RECON == WENO5)
+                weno5<R>(w[0].c[c], w[1].c[c], w[2].c[c], w[3].c[c], w[4].c[c], wL.c[c], wR.c[c]);
+            else
+                weno7<R>(w[0].c[c], w[1].c[c], w[2].c[c], w[3].c[c], w[4].c[c], w[5].c[c], w[6].c[c], wL.c[c],
+                         wR.c[c]);
+        }
     }
 }
 
@@ -658,7 +672,8 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
     __syncthreads();
     // B: primitive cell averages wS on the window (FP64, then cast)
     // WENO weights in fd's arithmetic if all of the window lies in its range
-    constexpr bool WENO_FD = RECON >= WENO3 && std::is_same<R, double>::value;
+    // (split precision, whose contracted last bits follow the form, keeps the general one)
+    constexpr bool WENO_FD = RECON >= WENO3 && std::is_same<R, double>::value && !SPLIT;
     bool wok = true;
     for (int i = threadIdx.x; i < NW; i += blockDim.x) {
         const int iq = e(bw + i) - bq;
@@ -1108,7 +1123,8 @@ void recon2d_kernel(SweepArgs a) {
     __syncthreads();
     // B: wS for s in [s0-4, s0+TS+4), own rows t in [t0, t0+TT)
     // WENO weights in fd's arithmetic if all of the window lies in its range
-    constexpr bool WENO_FD = RECON >= WENO3 && std::is_same<R, double>::value;
+    // (split precision, whose contracted last bits follow the form, keeps the general one)
+    constexpr bool WENO_FD = RECON >= WENO3 && std::is_same<R, double>::value && !SPLIT;
     bool wok = true;
     for (int i = threadIdx.x; i < TT * NWS; i += blockDim.x) {
         const int it = i / NWS, is = i % NWS;

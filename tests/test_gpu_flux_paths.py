@@ -308,3 +308,25 @@ def test_marching_llf_writes_the_last_interface_from_the_last_tile(shape, subgri
         assert torch.equal(f0, ref[0]["raw"]) and torch.equal(f1, ref[1]["raw"])
         assert eig == [ref[0]["eigmax"], ref[1]["eigmax"]]
     plan.close()
+
+
+SPLIT_WENO = {((60,), "weno3"): "87ec14056994", ((60,), "weno5"): "f6f5dbaacdd6", ((60,), "weno7"): "37495a2602b1",
+              ((19, 23), "weno3"): "28637c7286e8", ((19, 23), "weno5"): "ccc6b3d22937", ((19, 23), "weno7"): "6ec2d1575ab7"}
+
+
+@pytest.mark.parametrize("shape,subgrid", SPLIT_WENO, ids=str)
+def test_split_weno_keeps_its_rounding(shape, subgrid):
+    """Split precision contracts multiplications into additions, so that its
+    last bits follow the source form of the WENO weights: the fluxes' bytes
+    (SHA-256, zeros made positive) are those of the form it was brought up with."""
+    import hashlib
+    from astrea_amd.plan import Plan
+    dims = len(shape)
+    plan = Plan(dims, subgrid, "llf", "ssprk(3,3)",
+                [dict(n0=shape[0], n1=shape[1] if dims == 2 else 1, boundary="wrap", dx=1 / 64, gamma=1.4, cfl=.4, t_end=1e9)],
+                varmask=0x13 if dims == 1 else 0x17, precision="split")
+    plan.load([_grid(shape, 41)])
+    out = plan.evolve_space(0)
+    plan.close()
+    got = hashlib.sha256(b"".join((out[ax]["flux"] + 0.).tobytes() for ax in out)).hexdigest()
+    assert got.startswith(SPLIT_WENO[shape, subgrid])
