@@ -615,8 +615,9 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
     __shared__ R wl[RECON == PCM ? 1 : NV][RECON == PCM ? 1 : NC];
     __shared__ R wr[RECON == PCM ? 1 : NV][RECON == PCM ? 1 : NC];
     // only the Lax-Friedrichs and Lax-Wendroff solvers take a neighbour's radius;
-    // the others' own one is formed with their flux
-    constexpr bool MERGED = RECON != PCM && SOLVER != LLF && SOLVER != LW;
+    // the others' own one is formed with their flux (not in split precision,
+    // whose FP32 radius, contracted beside the flux, rounds otherwise than LLF's)
+    constexpr bool MERGED = RECON != PCM && SOLVER != LLF && SOLVER != LW && !SPLIT;
     __shared__ R rad[MERGED ? 1 : NR];
     // PPM forms face values of positions [s0-2, s0+TS+2) and curvatures of
     // [s0-3, s0+TS+5) once per position, in cq and qd; the fluxes take cq's
@@ -922,10 +923,7 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
                 g.fm = phys_flux<A, MASK, 0>(g.wm, A(gR));
                 g.fp = phys_flux<A, MASK, 0>(g.wp, A(gR));
             }
-            if constexpr (MERGED) {
-                if constexpr (SPLIT) rk = radius<MASK, 0, true>(jac_state<MASK, true, RECON != PLM>(f.wp, f.wm), gamma);
-                else rk = radius_of(arith, f.wp, f.wm);
-            }
+            if constexpr (MERGED) rk = radius_of(arith, f.wp, f.wm);
             F = cast8<R, A, MASK>(riemann<A, MASK, SOLVER, 0>(g, A(lam), sax, A(Bn), A(gR), 1, a.compat != 0, SPLIT, &ok));
         };
         if constexpr (FAST) {

@@ -330,3 +330,25 @@ def test_split_weno_keeps_its_rounding(shape, subgrid):
     plan.close()
     got = hashlib.sha256(b"".join((out[ax]["flux"] + 0.).tobytes() for ax in out)).hexdigest()
     assert got.startswith(SPLIT_WENO[shape, subgrid])
+
+
+@pytest.mark.parametrize("n", [60, 300, 700])
+@pytest.mark.parametrize("subgrid", ["plm", "ppm", "weno3", "weno5", "weno7"])
+def test_split_wave_speed_is_the_same_with_every_solver(n, subgrid):
+    """The 1D wave speed of a stage comes from its interface states alone:
+    split-precision HLLC, HLLD and LLF plans report the same one, bit for bit."""
+    from astrea_amd.plan import Plan
+    g = _grid((n,), 41, mhd=True)
+    g[..., 5] = .75
+    speed = {}
+    for solver, mask in (("llf", 0x13), ("hllc", 0x13), ("llf", 0xFF), ("hllc", 0xFF), ("hlld", 0xFF)):
+        q = g.copy()
+        if mask == 0x13:
+            q[..., 5:] = 0
+        plan = Plan(1, subgrid, solver, "ssprk(3,3)",
+                    [dict(n0=n, boundary="wrap", dx=1 / 64, gamma=1.4, cfl=.4, t_end=1e9)], varmask=mask, precision="split")
+        plan.load([q])
+        speed[solver, mask] = plan.evolve_space(0)[0]["eigmax"]
+        plan.close()
+    assert speed["hllc", 0x13] == speed["llf", 0x13]
+    assert speed["hllc", 0xFF] == speed["hlld", 0xFF] == speed["llf", 0xFF]
