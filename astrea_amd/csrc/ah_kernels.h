@@ -180,7 +180,10 @@ __device__ inline R flat_chi_at(const Acc& W, int flattener, int mm) {
 // WENO of one cell, every component, in arithmetic fd.  Two thirds of the issue
 // of its launch is the weights' divisions: fd takes WENO5 at 768^2 MHD from
 // 62/61 to 55/53 us per launch (x/y), at 517 x 333 from 15.0/16.6 to 13.5/14.4.
-template <class A, class R, int MASK, int RECON, class Acc>
+// The callers keep a loop for each arithmetic: a choice per cell lets the
+// compiler start every component's shared terms before it (WENO7 then took 256
+// registers and spilled, 192 1D problems 585 us per step where loops take 363).
+template <class R, int MASK, int RECON, class Acc>
 __device__ inline void weno_cell(const Acc& W, int ce, V8<R>& wL, V8<R>& wR) {
     constexpr int H = RECON == WENO3 ? 1 : (RECON == WENO5 ? 2 : 3);
     V8<R> w[2 * H + 1];
@@ -190,11 +193,11 @@ __device__ inline void weno_cell(const Acc& W, int ce, V8<R>& wL, V8<R>& wR) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
         if (!VS<MASK>::live(c)) continue;
-        A l, r;
-        auto x = [&](int k) { return A(w[k].c[c]); };
-        if constexpr (RECON == WENO3) weno3<A>(x(0), x(1), x(2), l, r);
-        else if constexpr (RECON == WENO5) weno5<A>(x(0), x(1), x(2), x(3), x(4), l, r);
-        else weno7<A>(x(0), x(1), x(2), x(3), x(4), x(5), x(6), l, r);
+        fd l, r;
+        auto x = [&](int k) { return fd(w[k].c[c]); };
+        if constexpr (RECON == WENO3) weno3<fd>(x(0), x(1), x(2), l, r);
+        else if constexpr (RECON == WENO5) weno5<fd>(x(0), x(1), x(2), x(3), x(4), l, r);
+        else weno7<fd>(x(0), x(1), x(2), x(3), x(4), x(5), x(6), l, r);
         wL.c[c] = R(l);
         wR.c[c] = R(r);
     }
@@ -786,6 +789,7 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
                                            [&](int v, int j) -> R& { return fc_s[v][j]; });
                 __syncthreads();
             }
+            auto each = [&](auto arith) {
             for (int i = threadIdx.x; i < NC; i += blockDim.x) {
                 V8<R> L, Rr;
                 if constexpr (TWO)
@@ -795,8 +799,8 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
                 else if constexpr (RECON == PPM)
                     recon_cell<R, MASK, RECON, 0>(Wc, Wc.e(bcl + i), a.limiter, a.flattener, L, Rr,
                                                   [&](int mm) { return chi_s[mm - (s0 - 3)]; });
-                else if (WENO_FD && wok)
-                    weno_cell<typename std::conditional<WENO_FD, fd, R>::type, R, MASK, RECON>(Wc, Wc.e(bcl + i), L, Rr);
+                else if constexpr (is_fd<decltype(arith)>)
+                    weno_cell<R, MASK, RECON>(Wc, Wc.e(bcl + i), L, Rr);
                 else
                     recon_cell<R, MASK, RECON, 0>(Wc, Wc.e(bcl + i), a.limiter, a.flattener, L, Rr);
 #pragma unroll
@@ -806,6 +810,12 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
                         wr[V::slot(c)][i] = Rr.c[c];
                     }
             }
+            };
+            if constexpr (WENO_FD) {
+                if (wok) each(fd(0.0));
+                else each(R(0));
+            } else
+                each(R(0));
         };
         if (clampC) recon_cells(std::true_type{});
         else recon_cells(std::false_type{});
@@ -1225,6 +1235,7 @@ void recon2d_kernel(SweepArgs a) {
         }
         __syncthreads();
     }
+    auto each = [&](auto arith) {
     for (int i = threadIdx.x; i < TT * TS; i += blockDim.x) {
         const int it = i / TS, is = i % TS;
         const int s = s0 + is, t = t0 + it;
@@ -1237,8 +1248,8 @@ void recon2d_kernel(SweepArgs a) {
         else if constexpr (RECON == PPM)
             recon_cell<R, MASK, RECON, AX>(W, s, a.limiter, a.flattener, L, Rr,
                                            [&](int mm) { return chi_s[it][mm - (s0 - 2)]; });
-        else if (WENO_FD && wok)
-            weno_cell<typename std::conditional<WENO_FD, fd, R>::type, R, MASK, RECON>(W, s, L, Rr);
+        else if constexpr (is_fd<decltype(arith)>)
+            weno_cell<R, MASK, RECON>(W, s, L, Rr);
         else
             recon_cell<R, MASK, RECON, AX>(W, s, a.limiter, a.flattener, L, Rr);
         const long long o = fo + (long long)t * ns + s;
@@ -1276,6 +1287,12 @@ void recon2d_kernel(SweepArgs a) {
             }
         }
     }
+    };
+    if constexpr (WENO_FD) {
+        if (wok) each(fd(0.0));
+        else each(R(0));
+    } else
+        each(R(0));
     };
     if (clampS) cells(std::true_type{});
     else cells(std::false_type{});
