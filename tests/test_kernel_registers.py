@@ -47,7 +47,7 @@ PLM, PPM, WENO3, WENO5, WENO7 = 1, 2, 3, 4, 5
 LLF, HLLC, HLLD = 0, 1, 2
 ROOM = [("recon2d", HYDRO2, (WENO3, WENO5, WENO7), (0, 1), 4), ("recon2d", MHD2, (WENO3, WENO5, WENO7), (0, 1), 3),
         ("sweep1d", HYDRO1, (WENO3, WENO5, WENO7), (LLF, HLLC), 4), ("sweep1d", ALL, (WENO3, WENO5), (LLF, HLLC), 3),
-        ("sweep1d", ALL, (WENO7,), (LLF, HLLC), 2)]
+        ("sweep1d", ALL, (WENO7,), (LLF, HLLC), 2), ("sweep1d", ALL, (PLM, WENO3), (HLLD,), 3)]
 
 
 @pytest.mark.parametrize("kernel,mask,recons,last,waves", ROOM, ids=str)
