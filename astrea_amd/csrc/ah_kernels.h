@@ -682,8 +682,11 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
     __syncthreads();
     // B: primitive cell averages wS on the window (FP64, then cast)
     // WENO weights in fd's arithmetic if all of the window lies in its range
-    // (split precision, whose contracted last bits follow the form, keeps the general one)
-    constexpr bool WENO_FD = RECON >= WENO3 && std::is_same<R, double>::value && !SPLIT;
+    // (split precision, whose contracted last bits follow the form, keeps the
+    // general one; so does WENO7 of eight components: beside the short weights
+    // the general ones run slower there, 64 tubes of 1601 cells LLF in range
+    // 126, out of it 148 us a step, where the general form alone takes 136)
+    constexpr bool WENO_FD = RECON >= WENO3 && std::is_same<R, double>::value && !SPLIT && !(RECON == WENO7 && V::MHD);
     bool wok = true;
     for (int i = threadIdx.x; i < NW; i += blockDim.x) {
         const int iq = e(bw + i) - bq;
