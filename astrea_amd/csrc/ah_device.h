@@ -818,7 +818,9 @@ __device__ inline HlldWave<double> wide(const HlldWave<R>& h) {
 // are the general ones.  From those ranges: fast speeds in [2^-31, 2^47], s - u
 // zero or in [2^-152, 2^49], the numerators of s_M and p* zero or in
 // [2^-416, 2^158].  With the checks that every divisor and rho* be at least
-// 2^-100 (dL, dR: 2^-150): s_M at most 2^212 and, as a multiple of 2^-466,
+// 2^-100 (dL, dR: zero, by which nothing is divided, or at least 2^-150; it is
+// zero where a field along the axis carries the fast wave, and 64 such tubes
+// PPM ran both forms, 122 us a step against 98): s_M at most 2^212 and, as a multiple of 2^-466,
 // s_M - u zero or at least that; rho* at most 2^179, dL at most 2^292; so every
 // quotient so far is zero or in [2^-758, 2^363] and its remainder a multiple of
 // 2^-571.  The numerators of the inner states are checked themselves: zero or at
@@ -872,8 +874,8 @@ __device__ inline HlldWave<R> hlld_wave(const V8<R>& wL, const V8<R>& wR, R Bn, 
     const R ps = gdiv_pos(rhoL * ptR * sLu - rhoR * ptL * sRu + rhoR * rhoL * sLu * sRu, den);
     const R Bn2 = Bn * Bn;
     const R dL = rhoL * sLu * sLM - Bn2, dR = rhoR * sRu * sRM - Bn2;
-    const R vqL = gdiv_pos(sM - uL, dL), vqR = gdiv_pos(sM - uR, dR);
-    const R BqL = gdiv_pos(rhoL * sq(sLu) - Bn2, dL), BqR = gdiv_pos(rhoR * sq(sRu) - Bn2, dR);
+    const R vqL = gdiv(sM - uL, dL), vqR = gdiv(sM - uR, dR);
+    const R BqL = gdiv(rhoL * sq(sLu) - Bn2, dL), BqR = gdiv(rhoR * sq(sRu) - Bn2, dR);
     HlldWave<R> h;
     // region select (solvers.py:226-231): regions 1 and 4 are the outer, 2 and 3
     // the inner states, 0 F(w-) and 5 F(w+); later masks overwrite earlier ones
@@ -922,7 +924,8 @@ __device__ inline HlldWave<R> hlld_wave(const V8<R>& wL, const V8<R>& wR, R Bn, 
     h.vB = hlld_dot<R, MASK>(v, B);
     if constexpr (is_fd<R>) {
         const double d1 = imin(imin_abs(den.v, sLM.v), imin(imin(rLs.v, rRs.v), ah_fabs(sRM.v)));
-        *ok = (d1 >= 0x1p-100) & (imin_abs(dL.v, dR.v) >= 0x1p-150) & (imin(discL.v, discR.v) >= 0.0) & (ex >= -799);
+        auto dok = [](double d) { return (ah_fabs(d) >= 0x1p-150) | (d == 0.0); };
+        *ok = (d1 >= 0x1p-100) & dok(dL.v) & dok(dR.v) & (imin(discL.v, discR.v) >= 0.0) & (ex >= -799);
     }
     return h;
 }
