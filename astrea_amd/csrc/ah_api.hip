@@ -74,50 +74,85 @@ bool author_supported(const ah_scheme* sch) {
            !sch->magnetic_2d && !sch->fuse2d && sch->tile_s == 0;
 }
 
-// Lines per tile of the marching flux launch, or 0 for the 2D flux tiles.
+// The 2D flux launch of a set of problems: as marching tiles of `lines` lines,
+// and whether those or the 2D tiles end sooner.
 //
 // A marching wave solves its own lines and two halo lines one after another,
 // so a launch takes about (rounds of resident waves) x (lines + 2) line times:
 // long tiles waste less on halo lines, short ones fill the chip.  The lines
 // are those with the least of that product; past two rounds the waves drain
 // unevenly and half a round is added for the tail.  Two hydrodynamic waves
-// (256 registers) or one MHD wave (504) fit a SIMD.
+// (256 registers) or one MHD wave (504) fit a SIMD, and a line takes less where
+// they do not share it.  A side counts by the waves it takes, so that narrow
+// problems, which leave lanes idle, pay for them.
 //
-// Below some cells the launch is one round of a few lines whatever they are,
-// and the tiles, whose four waves share one line's latency, end sooner.
-// Measured, us per launch (x + y sweep), tiles against marching: PPM/HLLC
-// 384^2 48 / 51, 512^2 63 / 62, 640^2 88 / 79, 1024^2 208 / 133; WENO5/LLF
-// 517 x 333 44 / 41, 512^2 PLM 52 / 45, 384^2 37 / 36; PLM/HLLD 384^2 87 / 82,
-// 512^2 124 / 110, 256^2 42 / 64.
-int march_lines_for(const ah_scheme& sch, int nprob, const ah_problem* probs, int cus, KernelSet* ks) {
-    if (sch.precision != AH_FP64 || sch.fuse2d || sch.ppm_author != AH_PPM_MC) return 0;
-    long long cells = 0;
-    for (int i = 0; i < nprob; ++i) {
-        if (probs[i].n0 <= 0 || probs[i].n1 <= 0) return 0;
-        cells += (long long)probs[i].n0 * probs[i].n1;
-    }
-    if (cells < (sch.solver == AH_LLF ? 160000 : 250000)) return 0;
-    if (!kernels_2d_march_fp64(sch.varmask, sch.recon, sch.solver, ks)) return 0;
-    const double slots = (ks->march_waves * 4) * (double)cus;
-    int best = 0;
-    double best_cost = 0.0;
-    for (int lines = 3; lines <= 24; ++lines) {
-        double cost = 0.0;
+// The tiles take a time of their own and one per tile, partly filled ones too.
+// The constants (us, of a card with 256 CUs) are fitted to both forms of
+// 26 sets of 1 to 1000 problems of 16 to 2048 cells a side; the choice then is
+// the faster one in all but three of 200 measurements, where it loses 3-11 %.
+// Measured, us per x + y sweep, tiles against marching: PPM/HLLC 384^2 47 / 51,
+// 512^2 65 / 69, 600^2 79 / 76, 1024^2 184 / 134, 64 x 64^2 69 / 79, 64 x 128^2
+// 207 / 184, 1000 x 16^2 74 / 116, 2 x 130000 297 / 427; PLM/LLF 512^2 53 / 48,
+// 1000 x 16^2 51 / 65; PLM/HLLD 300^2 62 / 74, 384^2 88 / 83, 512^2 128 / 108.
+struct FluxForm {
+    int lines = 0;  // 0: the tile form only
+    bool march = false;
+};
+
+FluxForm flux_form(const ah_scheme& sch, const KernelSet& ks, int cus, const std::vector<const ah_problem*>& probs) {
+    FluxForm form;
+    if (!ks.march[0]) return form;
+    // marching: a launch's own time, a line's, a line's with one wave on the SIMD; tiles: their own time, 1000 tiles'
+    struct Cost {
+        double m0, line, line1, t0, tiles;
+    };
+    static constexpr Cost PLM_COST[3] = {{8.6, 2.9, 1.8, 9.0, 9.4}, {9.6, 4.6, 2.5, 10.1, 11.3}, {11.3, 6.0, 6.0, 12.4, 25.8}};
+    static constexpr Cost HO_COST[3] = {{9.6, 3.3, 1.8, 9.4, 10.6}, {9.9, 5.1, 2.8, 10.7, 13.1}, {9.8, 6.3, 6.3, 11.0, 29.4}};
+    const int solver = sch.solver == AH_LLF ? 0 : sch.solver == AH_HLLC ? 1 : 2;
+    const Cost& k = (sch.recon == AH_PLM ? PLM_COST : HO_COST)[solver];
+    const double slots = (ks.march_waves * 4) * (double)cus;
+    double least = 0.0, march = 0.0, tiles = 0.0;
+    for (int lines = MARCH_LINES_MIN; lines <= MARCH_LINES_MAX; ++lines) {
+        double cost = 0.0, us = 0.0;
         for (int ax = 0; ax < 2; ++ax) {
             double waves = 0.0;
-            for (int i = 0; i < nprob; ++i) {
-                const int ns = ax == 0 ? probs[i].n0 : probs[i].n1, nt = ax == 0 ? probs[i].n1 : probs[i].n0;
-                waves += (double)((ns + ks->mw - 1) / ks->mw) * ((nt + lines - 1) / lines);
+            for (const ah_problem* q : probs) {
+                const int ns = ax == 0 ? q->n0 : q->n1, nt = ax == 0 ? q->n1 : q->n0;
+                waves += (double)((ns + ks.mw - 1) / ks.mw) * ((nt + lines - 1) / lines);
             }
             const double rounds = waves / slots;
-            cost += (rounds <= 2.0 ? (rounds <= 1.0 ? 1.0 : 2.0) : rounds + .5) * (lines + 2);
+            const double turns = (rounds <= 2.0 ? (rounds <= 1.0 ? 1.0 : 2.0) : rounds + .5) * (lines + 2);
+            cost += turns;
+            us += k.m0 + turns * (rounds <= .5 ? k.line1 : k.line);
         }
-        if (best == 0 || cost < best_cost) {
-            best = lines;
-            best_cost = cost;
+        if (form.lines == 0 || cost < least) {
+            form.lines = lines;
+            least = cost;
+            march = us;
         }
     }
-    return best;
+    for (int ax = 0; ax < 2; ++ax) {
+        double n = 0.0;
+        for (const ah_problem* q : probs) {
+            const int ns = ax == 0 ? q->n0 : q->n1, nt = ax == 0 ? q->n1 : q->n0;
+            n += (double)((ns + ks.fts[ax] - 1) / ks.fts[ax]) * ((nt + ks.ftt[ax] - 1) / ks.ftt[ax]);
+        }
+        tiles += k.t0 + k.tiles * 1e-3 * n * (256.0 / cus);
+    }
+    form.march = march <= tiles;
+    return form;
+}
+
+// a problem's marching tiles of one sweep, split evenly: no tile is left with a few cells or lines
+void march_tiles(const ah_problem& q, int ax, int lines, int width, int prob, std::vector<Tile>* out) {
+    const int ns = ax == 0 ? q.n0 : q.n1, nt = ax == 0 ? q.n1 : q.n0;
+    const int nw = (ns + width - 1) / width, nl = (nt + lines - 1) / lines;
+    for (int l = 0; l < nl; ++l)
+        for (int w = 0; w < nw; ++w) {
+            const int sb = (int)((long long)ns * w / nw), se = (int)((long long)ns * (w + 1) / nw);
+            const int tb = (int)((long long)nt * l / nl), te = (int)((long long)nt * (l + 1) / nl);
+            out->push_back({prob, sb, tb, march_pad(se - sb, te - tb)});
+        }
 }
 
 int popcount8(int m) {
@@ -151,8 +186,9 @@ struct ah_plan {
     int comb_cells = 256;        // cells per combination tile
     bool fold_finish = false;    // the last combination ends the step (few tiles per problem)
     // tile lists: 0 = 1D sweep, 1/2 = recon ax0/ax1, 3/4 = flux ax0/ax1, 5 = cells (combine),
-    // 6/7 = transverse reconstruction ax0/ax1 (MHD)
-    TileList tl[8];
+    // 6/7 = transverse reconstruction ax0/ax1 (MHD), 8/9 = marching flux ax0/ax1
+    TileList tl[10];
+    bool march = false;          // the flux launches take the marching form
     int max_blocks = 8192;  // grid cap per launch (workgroups loop over the tiles beyond it)
     // captured step graphs (ah_plan_step_graph)
     hipGraphExec_t graph_exec = nullptr;
@@ -358,10 +394,6 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
         case AH_SSPRK54: p->nregs = 5; break;
         case AH_SSPRK104: p->nregs = sch->magnetic_2d ? 4 : 3; break;  // + the refined increment
     }
-    // the marching flux launch where it is the faster form
-    const int march_lines = sch->dims == 2 ? march_lines_for(p->sch, nprob, probs, cus, &p->ks) : 0;
-    if (march_lines > 0)
-        for (int ax = 0; ax < 2; ++ax) p->ks.flux[ax] = p->ks.march[ax];
     // problem tables and tiles
     std::vector<ProbDesc> pd(nprob);
     // combination tiles: 256 cells (one per thread) in 1D, so the few large
@@ -376,10 +408,26 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
     for (int i = 0; i < nprob; ++i) {
         const ah_problem& q = probs[i];
         const int n1 = sch->dims == 1 ? 1 : q.n1;
-        if (q.n0 <= 0 || n1 <= 0 || q.dx <= 0 || q.checkpoints <= 0 || (q.boundary != AH_EDGE && q.boundary != AH_WRAP)) {
+        if (q.n0 > 0 && n1 > 0) total += (long long)q.n0 * n1;
+        if (q.n0 <= 0 || n1 <= 0 || q.dx <= 0 || q.checkpoints <= 0 ||
+            (q.boundary != AH_EDGE && q.boundary != AH_WRAP) || total >= (1ll << 31)) {
             delete p;
             return AH_ERR_INVALID;
         }
+    }
+    total = 0;
+    // the flux launches' form
+    FluxForm form;
+    if (sch->dims == 2 && sch->precision == AH_FP64 && !sch->fuse2d && sch->ppm_author == AH_PPM_MC &&
+        kernels_2d_march_fp64(sch->varmask, sch->recon, sch->solver, &p->ks)) {
+        std::vector<const ah_problem*> all;
+        for (const ah_problem& q : p->probs) all.push_back(&q);
+        form = flux_form(p->sch, p->ks, cus, all);
+    }
+    p->march = form.march;
+    for (int i = 0; i < nprob; ++i) {
+        const ah_problem& q = probs[i];
+        const int n1 = sch->dims == 1 ? 1 : q.n1;
         pd[i].n0 = q.n0;
         pd[i].n1 = n1;
         pd[i].bc = q.boundary;
@@ -402,15 +450,8 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
                 if (p->ks.recon[ax])  // no reconstruction launch when the flux tiles reconstruct
                     for (int t0 = 0; t0 < nt; t0 += p->ks.rtt[ax])
                         for (int s0 = 0; s0 < ns; s0 += p->ks.rts[ax]) p->tl[1 + ax].full.push_back({i, s0, t0, 0});
-                if (march_lines > 0) {
-                    // even splits: no tile is left with a few cells or lines
-                    const int nw = (ns + p->ks.mw - 1) / p->ks.mw, nl = (nt + march_lines - 1) / march_lines;
-                    for (int l = 0; l < nl; ++l)
-                        for (int w = 0; w < nw; ++w) {
-                            const int sb = (int)((long long)ns * w / nw), se = (int)((long long)ns * (w + 1) / nw);
-                            const int tb = (int)((long long)nt * l / nl), te = (int)((long long)nt * (l + 1) / nl);
-                            p->tl[3 + ax].full.push_back({i, sb, tb, march_pad(se - sb, te - tb)});
-                        }
+                if (form.march) {
+                    march_tiles(q, ax, form.lines, p->ks.mw, i, &p->tl[8 + ax].full);
                 } else
                     for (int t0 = 0; t0 < nt; t0 += p->ks.ftt[ax])
                         for (int s0 = 0; s0 < ns; s0 += p->ks.fts[ax]) p->tl[3 + ax].full.push_back({i, s0, t0, 0});
@@ -430,11 +471,7 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
     // on one address cost more than the separate end-of-step launch (1024^2:
     // 1024 tiles, +5 us against the launch's 5 us)
     p->fold_finish = !sch->magnetic_2d && max_ctiles <= 64;
-    if (total >= (1ll << 31)) {
-        delete p;
-        return AH_ERR_INVALID;
-    }
-    for (int l : {0, 1, 2, 3, 4, 6, 7}) xcd_order(p->tl[l].full);
+    for (int l : {0, 1, 2, 3, 4, 6, 7, 8, 9}) xcd_order(p->tl[l].full);
     bool up = hipMalloc((void**)&p->d_pd, nprob * sizeof(ProbDesc)) == hipSuccess &&
               hipMemcpy(p->d_pd, pd.data(), nprob * sizeof(ProbDesc), hipMemcpyHostToDevice) == hipSuccess &&
               hipMalloc((void**)&p->d_ps, nprob * sizeof(ProbState)) == hipSuccess &&
@@ -655,8 +692,9 @@ static void launch_space(ah_plan* p, const double* X, double* Lout, int stage0, 
             ProfScope ps_(p, ax == 0 ? AH_K_RECON0 : AH_K_RECON1, s);
             p->ks.recon[ax](a, blocks_for(p, p->tl[1 + ax]), s);
         }
-        a.tiles = p->tl[3 + ax].d;
-        a.ntiles_dev = p->tl[3 + ax].d_count;
+        const TileList& tl = p->tl[(p->march ? 8 : 3) + ax];
+        a.tiles = tl.d;
+        a.ntiles_dev = tl.d_count;
         a.last = ax == 1;
         a.out = ax == 0 ? p->Dbuf : Lout;
         if (ax == 0) a.fuse_k2 = nullptr;  // the first sweep writes its D
@@ -666,7 +704,7 @@ static void launch_space(ah_plan* p, const double* X, double* Lout, int stage0, 
         a.flux_plane = ax == 0 ? (long long)(p->probs[0].n0 + 1) * p->probs[0].n1
                                : (long long)(p->probs[0].n1 + 1) * p->probs[0].n0;
         ProfScope ps_(p, ax == 0 ? AH_K_FLUX0 : AH_K_FLUX1, s);
-        p->ks.flux[ax](a, blocks_for(p, p->tl[3 + ax]), s);
+        (p->march ? p->ks.march : p->ks.flux)[ax](a, blocks_for(p, tl), s);
     }
 }
 

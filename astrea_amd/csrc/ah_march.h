@@ -38,6 +38,9 @@ constexpr int march_width() { return SOLVER == LLF ? 62 : 63; }
 template <int MASK>
 constexpr int march_waves() { return VS<MASK>::MHD ? 1 : 2; }
 
+// lines of a tile
+constexpr int MARCH_LINES_MIN = 3, MARCH_LINES_MAX = 24;
+
 // Tile.pad of the marching kernel: own cells along the sweep, own lines
 constexpr int march_pad(int width, int lines) { return (lines << 8) | width; }
 

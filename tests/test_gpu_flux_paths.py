@@ -389,3 +389,90 @@ def test_hlld_with_a_field_along_the_sweep_that_carries_the_fast_wave(shape, sub
                 if s is not None:  # the energy flux does not scale (p* leaves a velocity out)
                     assert np.isfinite(f[..., i]).all()
                     assert np.array_equal(g[..., i], np.ldexp(f[..., i], s - 60)), (q, ax, i)
+
+
+def _smooth(shape, seed, mhd=False):
+    """Conservative state of order one with moderate waves only (and a field):
+    every interface is a weak one."""
+    r = np.random.default_rng(seed)
+    x, y = np.meshgrid(*((np.arange(n) + .5) / n for n in shape), indexing="ij")
+
+    def wave(a, kx, ky):
+        return a * np.sin(2 * np.pi * (kx * x + ky * y) + r.uniform(0, 2 * np.pi))
+    g = np.zeros(shape + (8,))
+    g[..., 0] = 1.2 + wave(.1, 1, 2)
+    v = [.2 + wave(.1, 1, 1), -.1 + wave(.1, 2, 1)]
+    b = [.3 + wave(.1, 0, 1), .25 + wave(.1, 1, 0)] if mhd else [0 * x, 0 * x]
+    for c in (0, 1):
+        g[..., 1 + c], g[..., 5 + c] = g[..., 0] * v[c], b[c]
+    g[..., 4] = (1. + wave(.1, 2, 1)) / .4 + .5 * (g[..., 0] * (v[0] ** 2 + v[1] ** 2) + b[0] ** 2 + b[1] ** 2)
+    return g
+
+
+FORMS = [("plm", "llf", "wrap"), ("ppm", "hllc", "edge"), ("weno5", "hllc", "wrap"), ("plm", "hlld", "edge"),
+         ("ppm", "hlld", "wrap"), ("weno5", "hlld", "edge"), ("weno5", "hlld", "wrap")]
+
+
+@pytest.mark.parametrize("subgrid,solver,boundary", FORMS)
+def test_narrow_problems_march_beside_a_large_one(subgrid, solver, boundary):
+    """Two steps of a batch that a large problem takes to the marching launch,
+    against each problem alone, which for all but the large one are the 2D
+    tiles: bit for bit, finite, and the state has moved."""
+    import torch
+    from astrea_amd.plan import Plan
+    mhd = solver == "hlld"
+    shapes = [(5, 7), (64, 63), (62, 126), (2, 9), (130, 33), (1, 50), (63, 64), (200, 3), (290, 280), (1100, 1000)]
+    probs = [dict(n0=a, n1=b, boundary=boundary, dx=1 / max(a, b), gamma=1.4, cfl=.3, t_end=1e9) for a, b in shapes]
+    grids = [torch.from_numpy(_smooth(s, 11 + i, mhd)).cuda() for i, s in enumerate(shapes)]
+
+    def run(ps, gs):
+        plan = Plan(2, subgrid, solver, "ssprk(3,3)", ps, varmask=0x77 if mhd else 0x17, magnetic_2d=mhd,
+                    compat="physical")
+        plan.load(gs)
+        plan.reset()
+        first = plan.state.clone()
+        plan.step(2)
+        out, st = plan.state.clone(), plan.status()
+        assert bool(torch.isfinite(out).all()) and not any(s["failed"] for s in st)
+        offs = plan.offsets + [plan.total]
+        plan.close()
+        return [out[:, offs[i]:offs[i + 1]] for i in range(len(ps))], st, first
+    both, st, first = run(probs, grids)
+    assert not torch.equal(torch.cat(both, 1), first)
+    for i in range(len(shapes) - 1):
+        (one,), (s1,), _ = run(probs[i:i + 1], grids[i:i + 1])
+        assert torch.equal(both[i], one), shapes[i]
+        assert st[i] == s1, shapes[i]
+
+
+def _flux_us(shapes, subgrid, solver):
+    """Time of a step's flux launches."""
+    import torch
+    from astrea_amd.plan import Plan
+    mhd = solver == "hlld"
+    probs = [dict(n0=a, n1=b, boundary="wrap", dx=1 / max(a, b), gamma=1.4, cfl=.3, t_end=1e9)
+             for a, b in shapes]
+    plan = Plan(2, subgrid, solver, "ssprk(3,3)", probs, varmask=0x77 if mhd else 0x17, magnetic_2d=mhd, compat="physical")
+    plan.load([torch.from_numpy(_smooth(s, 5, mhd)).cuda() for s in shapes])
+    plan.reset()
+    plan.step(2)
+    best = np.inf
+    for _ in range(4):
+        plan.profile(200)
+        plan.step(2)
+        best = min(best, sum(ms for kind, (ms, _) in plan.profile_read().items() if "flux" in kind) / 2 * 1e3)
+    plan.profile(0)
+    assert not any(s["failed"] for s in plan.status())
+    plan.close()
+    return best
+
+
+@pytest.mark.parametrize("subgrid,solver", [("ppm", "hllc"), ("plm", "hllc"), ("weno5", "hlld")])
+@pytest.mark.parametrize("shapes", [[(2, 130000)], [(16, 16)] * 1000], ids=["2x130000", "1000x16x16"])
+def test_narrow_problems_are_not_slower_for_being_many(shapes, subgrid, solver):
+    """Flux launches on sides that leave a wave's lanes idle: twice the cells
+    take at most 2.2 times as long (the marching launch, which a number of cells
+    alone once chose, took 2.6 to 3.0 times as long as the tiles of half)."""
+    half = [(2, 65000)] if len(shapes) == 1 else shapes[::2]
+    whole, part = _flux_us(shapes, subgrid, solver), _flux_us(half, subgrid, solver)
+    assert whole <= 2.2 * part, (whole, part)
