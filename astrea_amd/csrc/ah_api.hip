@@ -22,6 +22,7 @@ namespace {
 // the device so a captured graph stays valid when the list is compacted.
 struct TileList {
     std::vector<Tile> full;
+    size_t room = 0;  // tiles the device list has to hold where they are more than full's
     Tile* d = nullptr;
     int* d_count = nullptr;
     int count = 0;
@@ -144,15 +145,16 @@ FluxForm flux_form(const ah_scheme& sch, const KernelSet& ks, int cus, const std
 }
 
 // a problem's marching tiles of one sweep, split evenly: no tile is left with a few cells or lines
-void march_tiles(const ah_problem& q, int ax, int lines, int width, int prob, std::vector<Tile>* out) {
+int march_tiles(const ah_problem& q, int ax, int lines, int width, int prob, std::vector<Tile>* out) {
     const int ns = ax == 0 ? q.n0 : q.n1, nt = ax == 0 ? q.n1 : q.n0;
     const int nw = (ns + width - 1) / width, nl = (nt + lines - 1) / lines;
-    for (int l = 0; l < nl; ++l)
+    for (int l = 0; out && l < nl; ++l)
         for (int w = 0; w < nw; ++w) {
             const int sb = (int)((long long)ns * w / nw), se = (int)((long long)ns * (w + 1) / nw);
             const int tb = (int)((long long)nt * l / nl), te = (int)((long long)nt * (l + 1) / nl);
             out->push_back({prob, sb, tb, march_pad(se - sb, te - tb)});
         }
+    return nw * nl;
 }
 
 int popcount8(int m) {
@@ -186,13 +188,17 @@ struct ah_plan {
     int comb_cells = 256;        // cells per combination tile
     bool fold_finish = false;    // the last combination ends the step (few tiles per problem)
     // tile lists: 0 = 1D sweep, 1/2 = recon ax0/ax1, 3/4 = flux ax0/ax1, 5 = cells (combine),
-    // 6/7 = transverse reconstruction ax0/ax1 (MHD), 8/9 = marching flux ax0/ax1
+    // 6/7 = transverse reconstruction ax0/ax1 (MHD), 8/9 = marching flux ax0/ax1.
+    // A plan of several problems that starts on the marching launch holds both
+    // flux lists, of the same problems at any time: a captured step keeps its
+    // kernel, whichever form the plan launches by then.
     TileList tl[10];
+    int cus = 256;
     bool march = false;          // the flux launches take the marching form
     int max_blocks = 8192;  // grid cap per launch (workgroups loop over the tiles beyond it)
-    // captured step graphs (ah_plan_step_graph)
-    hipGraphExec_t graph_exec = nullptr;
-    int graph_steps = 0;
+    // captured step graphs (ah_plan_step_graph), one for each form of the flux launches
+    hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
+    int graph_steps[2] = {0, 0};
     // snapshots taken inside the step program (ah_plan_set_capture); ctl null: off
     CaptureArgs cap = {};
     // bound memory
@@ -237,6 +243,17 @@ void xcd_order(std::vector<Tile>& v) {
             if (s < n) o.push_back(v[s]);
         }
     v.swap(o);
+}
+
+hipError_t drop_graphs(ah_plan* p) {
+    hipError_t rc = hipSuccess;
+    for (hipGraphExec_t& g : p->graph_exec) {
+        if (!g) continue;
+        const hipError_t e = hipGraphExecDestroy(g);
+        g = nullptr;
+        if (e != hipSuccess) rc = e;
+    }
+    return rc;
 }
 
 struct ProfScope {
@@ -394,6 +411,7 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
         case AH_SSPRK54: p->nregs = 5; break;
         case AH_SSPRK104: p->nregs = sch->magnetic_2d ? 4 : 3; break;  // + the refined increment
     }
+    p->cus = cus;
     // problem tables and tiles
     std::vector<ProbDesc> pd(nprob);
     // combination tiles: 256 cells (one per thread) in 1D, so the few large
@@ -416,7 +434,8 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
         }
     }
     total = 0;
-    // the flux launches' form
+    // the flux launches' form; several problems keep the tiles beside the
+    // marching lists, for when the large ones have ended (ah_plan_compact)
     FluxForm form;
     if (sch->dims == 2 && sch->precision == AH_FP64 && !sch->fuse2d && sch->ppm_author == AH_PPM_MC &&
         kernels_2d_march_fp64(sch->varmask, sch->recon, sch->solver, &p->ks)) {
@@ -452,7 +471,10 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
                         for (int s0 = 0; s0 < ns; s0 += p->ks.rts[ax]) p->tl[1 + ax].full.push_back({i, s0, t0, 0});
                 if (form.march) {
                     march_tiles(q, ax, form.lines, p->ks.mw, i, &p->tl[8 + ax].full);
-                } else
+                    // (fewer problems may take fewer lines a tile)
+                    p->tl[8 + ax].room += march_tiles(q, ax, MARCH_LINES_MIN, p->ks.mw, i, nullptr);
+                }
+                if (!form.march || nprob > 1)
                     for (int t0 = 0; t0 < nt; t0 += p->ks.ftt[ax])
                         for (int s0 = 0; s0 < ns; s0 += p->ks.fts[ax]) p->tl[3 + ax].full.push_back({i, s0, t0, 0});
                 if (sch->magnetic_2d)
@@ -481,10 +503,11 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
     for (TileList& L : p->tl) {
         if (!up) break;
         L.count = (int)L.full.size();
+        if (!L.count && (&L == p->tl + 3 || &L == p->tl + 4 || &L >= p->tl + 8)) continue;  // a flux form not launched
         up = hipMalloc((void**)&L.d_count, sizeof(int)) == hipSuccess &&
              hipMemcpy(L.d_count, &L.count, sizeof(int), hipMemcpyHostToDevice) == hipSuccess;
         if (up && L.count)
-            up = hipMalloc((void**)&L.d, L.full.size() * sizeof(Tile)) == hipSuccess &&
+            up = hipMalloc((void**)&L.d, std::max(L.full.size(), L.room) * sizeof(Tile)) == hipSuccess &&
                  hipMemcpy(L.d, L.full.data(), L.full.size() * sizeof(Tile), hipMemcpyHostToDevice) == hipSuccess;
     }
     // 32 workgroups per CU: a 1024^2 grid's sweeps then launch one workgroup
@@ -504,7 +527,7 @@ int ah_plan_destroy(ah_plan* p) {
     if (!p) return AH_ERR_INVALID;
     for (hipEvent_t e : p->ev) (void)hipEventDestroy(e);
     int rc = AH_OK;
-    if (p->graph_exec && hipGraphExecDestroy(p->graph_exec) != hipSuccess) rc = AH_ERR_HIP;
+    if (drop_graphs(p) != hipSuccess) rc = AH_ERR_HIP;
     void* bufs[] = {p->d_pd, p->d_ps, p->d_done};
     for (void* b : bufs)
         if (b && hipFree(b) != hipSuccess) rc = AH_ERR_HIP;
@@ -551,11 +574,7 @@ int ah_plan_bind(ah_plan* p, double* state, void* ws, size_t ws_bytes) {
     ah_plan_workspace_size(p, &need);
     if (ws_bytes < need) return AH_ERR_NOMEM;
     // a captured step graph holds the previously bound buffers
-    if (p->graph_exec) {
-        HIPCHK(hipGraphExecDestroy(p->graph_exec));
-        p->graph_exec = nullptr;
-        p->graph_steps = 0;
-    }
+    HIPCHK(drop_graphs(p));
     char* c = (char*)ws;
     p->U = state;
     p->regs[0] = state;
@@ -623,6 +642,7 @@ int ah_plan_reset(ah_plan* p, void* stream) {
         HIPCHK(hipMemcpy(L.d, L.full.data(), L.full.size() * sizeof(Tile), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(L.d_count, &L.count, sizeof(int), hipMemcpyHostToDevice));
     }
+    p->march = !p->tl[8].full.empty();
     hipLaunchKernelGGL(reset_kernel, dim3((p->nprob + 255) / 256), dim3(256), 0, s, p->d_pd, p->d_ps, p->nprob);
     HIPCHK(hipGetLastError());
     return AH_OK;
@@ -973,10 +993,11 @@ int ah_plan_step_graph(ah_plan* p, int nsteps, int nlaunch, void* stream) {
     if (!p || nsteps <= 0 || nlaunch < 0 || !stream) return AH_ERR_INVALID;
     if (!p->bound) return AH_ERR_STATE;
     hipStream_t s = (hipStream_t)stream;
-    if (!p->graph_exec || p->graph_steps != nsteps) {
-        if (p->graph_exec) {
-            HIPCHK(hipGraphExecDestroy(p->graph_exec));
-            p->graph_exec = nullptr;
+    hipGraphExec_t& exec = p->graph_exec[p->march];
+    if (!exec || p->graph_steps[p->march] != nsteps) {
+        if (exec) {
+            HIPCHK(hipGraphExecDestroy(exec));
+            exec = nullptr;
         }
         std::vector<hipEvent_t> saved;
         saved.swap(p->ev);  // no event records inside a captured graph
@@ -986,15 +1007,15 @@ int ah_plan_step_graph(ah_plan* p, int nsteps, int nlaunch, void* stream) {
         const hipError_t e1 = hipStreamEndCapture(s, &g);
         saved.swap(p->ev);
         if (e1 != hipSuccess || !g) return AH_ERR_HIP;
-        const hipError_t e2 = hipGraphInstantiate(&p->graph_exec, g, nullptr, nullptr, 0);
+        const hipError_t e2 = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         if (e2 != hipSuccess) {
-            p->graph_exec = nullptr;
+            exec = nullptr;
             return AH_ERR_HIP;
         }
-        p->graph_steps = nsteps;
+        p->graph_steps[p->march] = nsteps;
     }
-    for (int i = 0; i < nlaunch; ++i) HIPCHK(hipGraphLaunch(p->graph_exec, s));
+    for (int i = 0; i < nlaunch; ++i) HIPCHK(hipGraphLaunch(exec, s));
     return AH_OK;
 }
 
@@ -1044,11 +1065,7 @@ int ah_plan_set_capture(ah_plan* p, int prob, int mode, double* ring, int slots,
     if (mode != AH_CAPTURE_OFF && (!ring || !times || !ctl || slots <= 0)) return AH_ERR_INVALID;
     if (!p->bound) return AH_ERR_STATE;
     // a captured step graph holds the previous capture arguments
-    if (p->graph_exec) {
-        HIPCHK(hipGraphExecDestroy(p->graph_exec));
-        p->graph_exec = nullptr;
-        p->graph_steps = 0;
-    }
+    HIPCHK(drop_graphs(p));
     memset(&p->cap, 0, sizeof(p->cap));
     if (mode == AH_CAPTURE_OFF) return AH_OK;
     const ah_problem& q = p->probs[prob];
@@ -1075,12 +1092,32 @@ int ah_plan_compact(ah_plan* p, int* nactive, void* stream) {
     int na = 0;
     for (const ProbState& q : h) na += q.active ? 1 : 0;
     if (nactive) *nactive = na;
-    for (TileList& L : p->tl) {
+    // The marching lists are split anew for the problems left, and the 2D tiles
+    // take over where they are the faster form: in tiles of the lines that suit
+    // a large problem, the small ones it leaves behind are a few long waves.
+    // Four 128^2 PPM/HLLC problems after a 1024^2 one, us a step: 305 in its
+    // lines, 155 so; six 400^2 MHD ones down to one 1160, 587.  The first
+    // step graph after the turn is a new one, 0.3 ms for 16 steps.
+    FluxForm form;
+    if (!p->tl[8].full.empty() && na > 0) {
+        std::vector<const ah_problem*> left;
+        for (int i = 0; i < p->nprob; ++i)
+            if (h[i].active) left.push_back(&p->probs[i]);
+        form = flux_form(p->sch, p->ks, p->cus, left);
+        p->march = form.march || p->tl[3].full.empty();
+    }
+    for (int l = 0; l < 10; ++l) {
+        TileList& L = p->tl[l];
         if (L.full.empty()) continue;
         std::vector<Tile> act;
         act.reserve(L.full.size());
-        for (const Tile& t : L.full)
-            if (h[t.prob].active) act.push_back(t);
+        if (l >= 8 && na > 0 && na < p->nprob) {
+            for (int i = 0; i < p->nprob; ++i)
+                if (h[i].active) march_tiles(p->probs[i], l - 8, form.lines, p->ks.mw, i, &act);
+            xcd_order(act);
+        } else
+            for (const Tile& t : L.full)
+                if (h[t.prob].active) act.push_back(t);
         L.count = (int)act.size();
         if (L.count) HIPCHK(hipMemcpy(L.d, act.data(), act.size() * sizeof(Tile), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(L.d_count, &L.count, sizeof(int), hipMemcpyHostToDevice));
@@ -1091,10 +1128,7 @@ int ah_plan_compact(ah_plan* p, int* nactive, void* stream) {
 int ah_plan_set_blocks(ah_plan* p, int max_blocks) {
     if (!p || max_blocks <= 0) return AH_ERR_INVALID;
     p->max_blocks = max_blocks;
-    if (p->graph_exec) {
-        HIPCHK(hipGraphExecDestroy(p->graph_exec));
-        p->graph_exec = nullptr;
-    }
+    HIPCHK(drop_graphs(p));
     return AH_OK;
 }
 

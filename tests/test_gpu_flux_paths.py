@@ -445,17 +445,56 @@ def test_narrow_problems_march_beside_a_large_one(subgrid, solver, boundary):
         assert st[i] == s1, shapes[i]
 
 
-def _flux_us(shapes, subgrid, solver):
-    """Time of a step's flux launches."""
+@pytest.mark.parametrize("subgrid,solver", [("ppm", "hllc"), ("plm", "llf"), ("weno5", "hlld")])
+def test_a_batch_keeps_its_bits_when_large_problems_end(subgrid, solver):
+    """A batch whose problems end one after another, largest first, so that its
+    flux launches split anew and then turn to the 2D tiles; twice from the
+    start, the second time with the graphs of the first."""
+    import torch
+    from astrea_amd import batch
+    from astrea_amd.plan import Plan
+    mhd = solver == "hlld"
+    shapes, steps = [(1100, 1000), (700, 650), (128, 100), (64, 300)], [2, 5, 11, 16]
+    probs = [dict(n0=a, n1=b, boundary="wrap", dx=1 / 512, gamma=1.4, cfl=.3, t_end=1e9, max_steps=k)
+             for (a, b), k in zip(shapes, steps)]
+    grids = [torch.from_numpy(_smooth(s, 5 + i, mhd)).cuda() for i, s in enumerate(shapes)]
+
+    def run(ps, gs, use_graph, times):
+        plan = Plan(2, subgrid, solver, "ssprk(3,3)", ps, varmask=0x77 if mhd else 0x17, magnetic_2d=mhd,
+                    compat="physical")
+        out = []
+        for _ in range(times):
+            plan.load(gs)
+            plan.reset()
+            torch.cuda.synchronize()
+            st, _, _ = batch.run(plan, chunk=2, use_graph=use_graph)
+            out.append((plan.state.clone(), st))
+        offs = plan.offsets + [plan.total]
+        plan.close()
+        return out, offs
+    runs, offs = run(probs, grids, True, 2)
+    runs += run(probs, grids, False, 1)[0]
+    for i, k in enumerate(steps):
+        (one, (s1,)), = run(probs[i:i + 1], grids[i:i + 1], False, 1)[0]
+        assert s1["steps"] == k and not s1["failed"] and bool(torch.isfinite(one).all())
+        for state, st in runs:
+            assert torch.equal(state[:, offs[i]:offs[i + 1]], one), shapes[i]
+            assert st[i] == s1
+
+
+def _flux_us(shapes, subgrid, solver, ends=None):
+    """Time of a step's flux launches, after the problems with an end have reached it."""
     import torch
     from astrea_amd.plan import Plan
     mhd = solver == "hlld"
-    probs = [dict(n0=a, n1=b, boundary="wrap", dx=1 / max(a, b), gamma=1.4, cfl=.3, t_end=1e9)
-             for a, b in shapes]
+    probs = [dict(n0=a, n1=b, boundary="wrap", dx=1 / max(a, b), gamma=1.4, cfl=.3, t_end=1e9,
+                  max_steps=(ends[i] if ends else -1)) for i, (a, b) in enumerate(shapes)]
     plan = Plan(2, subgrid, solver, "ssprk(3,3)", probs, varmask=0x77 if mhd else 0x17, magnetic_2d=mhd, compat="physical")
     plan.load([torch.from_numpy(_smooth(s, 5, mhd)).cuda() for s in shapes])
     plan.reset()
     plan.step(2)
+    if ends:
+        plan.compact()
     best = np.inf
     for _ in range(4):
         plan.profile(200)
@@ -465,6 +504,16 @@ def _flux_us(shapes, subgrid, solver):
     assert not any(s["failed"] for s in plan.status())
     plan.close()
     return best
+
+
+@pytest.mark.parametrize("subgrid,solver", [("ppm", "hllc"), ("plm", "llf"), ("weno5", "hlld")])
+def test_a_small_problem_is_as_fast_beside_large_ones_that_have_ended(subgrid, solver):
+    """The flux launches of a 96^2 problem left of a batch take the time of that
+    problem alone (both forms' lines for the 2048^2 one took 2.4 to 3.2 times
+    it), and 3/2 of it at most."""
+    alone = _flux_us([(96, 96)], subgrid, solver)
+    left = _flux_us([(2048, 2048), (96, 96)], subgrid, solver, ends=[2, -1])
+    assert left <= 1.5 * alone, (left, alone)
 
 
 @pytest.mark.parametrize("subgrid,solver", [("ppm", "hllc"), ("plm", "hllc"), ("weno5", "hlld")])
