@@ -272,6 +272,17 @@ struct ProfScope {
 }  // namespace
 
 namespace {
+// Whether a snapshot takes the tiles: in small ones the tiles' barriers are all
+// that counts, and a thin domain leaves most of each tile idle (and converted
+// for nothing where a window is).  us, a thread per cell / tiles: PPM 128^2
+// 4.0 / 4.3, 160^2 4.9 / 4.4, 512^2 13.3 / 7.3, 70000 x 2 8.6 / 32.4, 30000 x 12
+// 14.8 / 17.1, 9000 x 40 15.1 / 12.8 (MHD 17.9 / 19.5), 700 x 100 6.3 / 5.2; PLM
+// 30000 x 12 11.8 / 8.2, 70000 x 2 6.1 / 13.4; 1D PPM 32768 cells 3.4 / 3.6,
+// 131072 5.8 / 4.2 (MHD 7.7 / 6.3).
+bool snapshot_tiled(int dims, bool ho, long long cells, long long tiles) {
+    return cells >= (dims == 1 ? 100000 : 24000) && 512 * tiles <= (ho ? 3 : 6) * cells;
+}
+
 template <int MASK>
 void launch_snapshot(const ah_plan* p, int prob, double* out, hipStream_t s, const CaptureArgs& cap) {
     const ah_problem& q = p->probs[prob];
@@ -279,18 +290,22 @@ void launch_snapshot(const ah_plan* p, int prob, double* out, hipStream_t s, con
     const int bc = q.boundary == AH_WRAP ? WRAP : EDGE;
     const bool ho = p->sch.recon == AH_PPM || p->sch.recon == AH_WENO3 || p->sch.recon == AH_WENO5 ||
                     p->sch.recon == AH_WENO7;
+    const long long cells = (long long)q.n0 * n1, off = p->offs[prob];
     // the kernel's tiles (256 cells in 1D)
     const long long tiles = p->sch.dims == 1
                                 ? (q.n0 + 255) / 256
                                 : (long long)((q.n0 + SNAP_TI - 1) / SNAP_TI) * ((n1 + SNAP_TJ - 1) / SNAP_TJ);
-    const dim3 g((unsigned)tiles), b(256);
-    const long long off = p->offs[prob];
+    const bool tiled = snapshot_tiled(p->sch.dims, ho, cells, tiles);
+    const dim3 g((unsigned)(tiled ? tiles : (cells + 255) / 256)), b(256);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, g, b, 0, s, p->U, p->total, off, q.n0, n1, bc, q.gamma, out, cap);
+    };
     if (p->sch.dims == 1) {
-        if (ho) hipLaunchKernelGGL((snapshot_kernel<MASK, 1, true>), g, b, 0, s, p->U, p->total, off, q.n0, n1, bc, q.gamma, out, cap);
-        else hipLaunchKernelGGL((snapshot_kernel<MASK, 1, false>), g, b, 0, s, p->U, p->total, off, q.n0, n1, bc, q.gamma, out, cap);
+        if (tiled) ho ? launch(snapshot_kernel<MASK, 1, true>) : launch(snapshot_kernel<MASK, 1, false>);
+        else ho ? launch(snapshot_cells_kernel<MASK, 1, true>) : launch(snapshot_cells_kernel<MASK, 1, false>);
     } else {
-        if (ho) hipLaunchKernelGGL((snapshot_kernel<MASK, 2, true>), g, b, 0, s, p->U, p->total, off, q.n0, n1, bc, q.gamma, out, cap);
-        else hipLaunchKernelGGL((snapshot_kernel<MASK, 2, false>), g, b, 0, s, p->U, p->total, off, q.n0, n1, bc, q.gamma, out, cap);
+        if (tiled) ho ? launch(snapshot_kernel<MASK, 2, true>) : launch(snapshot_kernel<MASK, 2, false>);
+        else ho ? launch(snapshot_cells_kernel<MASK, 2, true>) : launch(snapshot_cells_kernel<MASK, 2, false>);
     }
 }
 

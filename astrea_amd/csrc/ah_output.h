@@ -31,6 +31,48 @@ __device__ inline bool capture_due(const CaptureArgs& c) {
     return st.steps != c.ctl[1] && (c.mode == 1 || st.ckpt != 0) && st.t <= c.t_end;
 }
 
+// One thread per cell, for snapshots of which that latency is all there is.
+template <int MASK, int DIM, bool HO>
+__global__ __launch_bounds__(256) void snapshot_cells_kernel(const double* X, long long P, long long off, int n0,
+                                                             int n1, int bc, double gamma, double* out,
+                                                             CaptureArgs cap) {
+    using V = VS<MASK>;
+    const long long cells = (long long)n0 * n1;
+    const long long cell = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (cell >= cells) return;
+    if (cap.ctl) {
+        if (!capture_due(cap)) return;
+        out = cap.ring + (cap.ctl[0] % cap.slots) * cells * 8;
+    }
+    const int i = (int)(cell / n1), j = (int)(cell % n1);
+    auto Q = [&](int ii, int jj) {
+        V8<double> q = zero8<double, MASK>();
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+            if (V::live(c)) q.c[c] = X[V::slot(c) * P + off + (long long)ii * n1 + jj];
+        return q;
+    };
+    const V8<double> q0 = Q(i, j);
+    V8<double> w;
+    if constexpr (HO) {
+        const int im = bcmap(i - 1, n0, bc), ip = bcmap(i + 1, n0, bc);
+        const V8<double> qxm = Q(im, j), qxp = Q(ip, j);
+        V8<double> qym = zero8<double, MASK>(), qyp = qym;
+        if constexpr (DIM == 2) {
+            qym = Q(i, bcmap(j - 1, n1, bc));
+            qyp = Q(i, bcmap(j + 1, n1, bc));
+        }
+        w = ho_cell_prim<MASK, DIM, false>(q0, qxm, qxp, qym, qyp, c2p<MASK, false>(q0, gamma),
+                                           c2p<MASK, false>(qxm, gamma), c2p<MASK, false>(qxp, gamma),
+                                           c2p<MASK, false>(qym, gamma), c2p<MASK, false>(qyp, gamma), gamma);
+    } else {
+        w = c2p<MASK, false>(q0, gamma);
+    }
+    const long long o = DIM == 2 ? ((long long)j * n0 + i) * 8 : (long long)i * 8;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) out[o + c] = V::live(c) ? w.c[c] : 0.0;
+}
+
 // One workgroup per tile of 8 x 32 cells (2D) or 256 cells (1D).  The state is
 // read along its rows, the snapshot is written along its own, transposed ones,
 // eight values a cell: the tile's primitives are turned in LDS and written as

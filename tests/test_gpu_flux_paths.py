@@ -525,3 +525,43 @@ def test_narrow_problems_are_not_slower_for_being_many(shapes, subgrid, solver):
     half = [(2, 65000)] if len(shapes) == 1 else shapes[::2]
     whole, part = _flux_us(shapes, subgrid, solver), _flux_us(half, subgrid, solver)
     assert whole <= 2.2 * part, (whole, part)
+
+
+@pytest.mark.parametrize("shape", [(160, 160), (161, 159), (159, 161), (7, 3500), (3400, 31), (100001,), (100352,)], ids=str)
+@pytest.mark.parametrize("subgrid,boundary", [("ppm", "wrap"), ("ppm", "edge"), ("plm", "edge")])
+def test_large_snapshots_at_tile_edges_and_unaligned_buffers(shape, subgrid, boundary):
+    """Snapshots large enough for the tiled conversion, of whole tiles and one
+    cell more or less, against the oracle's conversion of the same state."""
+    test_snapshot_at_tile_edges_and_unaligned_buffers(shape, subgrid, boundary)
+
+
+def _snapshot_us(shape, subgrid, mhd):
+    import torch
+    from astrea_amd.plan import Plan
+    dims = len(shape)
+    plan = Plan(dims, subgrid, "llf", "euler", [dict(n0=shape[0], n1=shape[1] if dims == 2 else 1, boundary="wrap", dx=.1,
+                                                     gamma=1.4, cfl=.4, t_end=1.)],
+                varmask=(0xFF if mhd else 0x13) if dims == 1 else (0x77 if mhd else 0x17))
+    plan.load([torch.ones(shape + (8,), dtype=torch.float64, device="cuda")
+               * torch.tensor([1., .1] + (dims == 2) * [.1] + (dims == 1) * [0.] + [0., 3.] + 3 * [0.], device="cuda")])
+    out = plan.snapshot(0)
+    best = np.inf
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(40):
+            plan.snapshot(0, out=out)
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) / 40 * 1e3)
+    plan.close()
+    return best
+
+
+@pytest.mark.parametrize("subgrid,mhd", [("ppm", False), ("ppm", True), ("plm", False)])
+def test_thin_snapshots_do_not_pay_for_whole_tiles(subgrid, mhd):
+    """The snapshot of a domain two cells high takes at most twice the time of
+    the same cells in a square (the tiles, which it fills to a sixteenth, took 3
+    to 8 times)."""
+    thin, square = _snapshot_us((70000, 2), subgrid, mhd), _snapshot_us((374, 374), subgrid, mhd)
+    assert thin <= 2 * square, (thin, square)
