@@ -81,7 +81,8 @@ __device__ inline bool ah_isfinite(float x) { return __builtin_isfinite(x); }
 // v_div_scale_f64 and one the 8-cycle v_div_fmas_f64); its square root scales
 // and classifies around v_rsq_f64 with two residual corrections (23 slots).
 // With operands and results far from the ends of the exponent range the
-// scalings are by one, so the refinement alone gives the same bits: 11 slots a
+// scalings are by one, so the refinement alone gives the same bits (but for the
+// sign of a zero quotient, which is always plus): 11 slots a
 // division (3 when the divisor's reciprocal is already there -- the sequence
 // is plain arithmetic on the divisor, which the compiler shares between
 // quotients), 14 a square root, and no branch between independent chains.
@@ -258,17 +259,18 @@ __device__ inline R dot_vB(const V8<R>& w) {
     return acc;
 }
 
-// Whether the arithmetic of fd is exact on what the solvers form
-// from two primitive states: density and pressure in [2^-60, 2^60], velocities
-// zero or in [2^-100, 2^60].  Differences and averages of such values are zero
-// or at least 2^-210, wave speeds and their differences zero or at least
-// 2^-440, the numerators of the HLLC speeds zero or at least 2^-703 and their
-// quotients at most 2^900: every remainder a division or square root corrects
-// with is a normal number (>= 2^-969 before the correction).  With a magnetic
-// field: density and pressure in [2^-30, 2^30], velocities and fields zero or in
-// [2^-100, 2^30]; hlld_wave checks what its longer chains make of them.
+// Whether the arithmetic of fd is exact on what the solvers form from two
+// primitive states: an adiabatic index in (1, 16] (the divisor gamma - 1 is then
+// at least 2^-52, and squared sound speeds are positive), density and pressure in
+// [2^-60, 2^60], velocities zero or in [2^-100, 2^60].  Differences and averages
+// of such values are zero or at least 2^-210, wave speeds and their differences
+// zero or at least 2^-440, the numerators of the HLLC speeds zero or at least
+// 2^-703 and their quotients at most 2^900: every remainder a division or square
+// root corrects with is a normal number (>= 2^-969 before the correction).  With a
+// magnetic field: density and pressure in [2^-30, 2^30], velocities and fields zero
+// or in [2^-100, 2^30]; hlld_wave checks what its longer chains make of them.
 template <int MASK>
-__device__ inline bool safe_states(const V8<double>& a, const V8<double>& b) {
+__device__ inline bool safe_states(const V8<double>& a, const V8<double>& b, double gamma) {
     using V = VS<MASK>;
     constexpr double HI = V::MHD ? 0x1p30 : 0x1p60, LO = V::MHD ? 0x1p-30 : 0x1p-60;
     double sum = (a.c[0] + b.c[0]) + (a.c[4] + b.c[4]);  // NaN and infinities fail the comparison
@@ -281,7 +283,7 @@ __device__ inline bool safe_states(const V8<double>& a, const V8<double>& b) {
             ex = min(ex, min(ea, eb));  // 0 for a zero
         }
     const double low = __builtin_fmin(__builtin_fmin(a.c[0], b.c[0]), __builtin_fmin(a.c[4], b.c[4]));
-    return sum <= HI && low >= LO && ex >= -99;
+    return sum <= HI && low >= LO && ex >= -99 && gamma > 1.0 && gamma <= 16.0;
 }
 // the same for a normal field
 __device__ inline bool safe_field(double Bn) { return ah_fabs(Bn) <= 0x1p30 && __builtin_amdgcn_frexp_exp(Bn) >= -99; }

@@ -878,7 +878,7 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
             const V8<R> wp = WL(je), wm = WR(je - 1);
             if constexpr (SPLIT) st = jac_state<MASK, true, RECON != PLM>(wp, wm);
             else if constexpr (FAST) {
-                if (__all(safe_states<MASK>(wp, wm))) r = radius_of(fd(0.0), wp, wm);
+                if (__all(safe_states<MASK>(wp, wm, gamma))) r = radius_of(fd(0.0), wp, wm);
                 else r = radius_of(R(0), wp, wm);
             } else st = (RECON == PLM) ? arith_avg<R, MASK>(wp, wm) : roe_avg<R, MASK>(wp, wm);
         }
@@ -946,7 +946,7 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
             F = cast8<R, A, MASK>(riemann<A, MASK, SOLVER, 0>(g, A(lam), sax, A(Bn), A(gR), 1, a.compat != 0, SPLIT, &ok));
         };
         if constexpr (FAST) {
-            ok = safe_states<MASK>(f.wm, f.wp);
+            ok = safe_states<MASK>(f.wm, f.wp, gamma);
             if constexpr (V::MHD) ok = ok && safe_field(Bn);
             const bool fast = __all(ok);
             if (fast) solve(fd(0.0));
@@ -1446,7 +1446,7 @@ void flux2d_kernel(SweepArgs a) {
                             xm.c[c] = pfm[j][V::slot(c)];
                             xp.c[c] = pfp[j][V::slot(c)];
                         }
-                    safe = safe && safe_states<MASK>(xm, xp);
+                    safe = safe && safe_states<MASK>(xm, xp, pd.gamma);
                 }
 #pragma unroll
                 for (int v = 0; v < NV; ++v) {

@@ -162,14 +162,14 @@ void flux2d_march_kernel(SweepArgs a) {
         }
         dwm = sub8<MASK>(wm, lm);
         dwp = sub8<MASK>(wp, lp);
-        if constexpr (FAST) okl = __all(safe_states<MASK>(lm, lp));
+        if constexpr (FAST) okl = __all(safe_states<MASK>(lm, lp, gamma));
     }
     MarchLine<MASK> x;      // face-averaged quantities of the line before
     V8<double> cwm, cwp;    // corrected interface states of the line before
     Wave wavx;              // HLLC, HLLD: the waves of its second solve in their place
     double lamx = 0.0, bnx = 0.0, lmax = 0.0;
     bool bad = false;
-    if constexpr (FAST) okw = __all(safe_states<MASK>(wm, wp));
+    if constexpr (FAST) okw = __all(safe_states<MASK>(wm, wp, gamma));
 #pragma unroll 1
     for (int c = c0; c <= t1; ++c) {
         MarchLine<MASK> y;
@@ -272,9 +272,9 @@ void flux2d_march_kernel(SweepArgs a) {
             };
             bool fast = false;
             if constexpr (FAST) {
-                const bool okh = __all(safe_states<MASK>(hm, hp));
+                const bool okh = __all(safe_states<MASK>(hm, hp, gamma));
                 fast = okl && okw && okh;
-                if constexpr (V::MHD) fast = fast && __all(safe_states<MASK>(ywm, ywp) && safe_field(bny));
+                if constexpr (V::MHD) fast = fast && __all(safe_states<MASK>(ywm, ywp, gamma) && safe_field(bny));
                 else fast = fast && __all(safe_derived(ywm, ywp));
                 okl = okw;
                 okw = okh;
