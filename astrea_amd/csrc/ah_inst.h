@@ -12,6 +12,16 @@ inline void set1d(KernelSet* ks) {
     // nearly empty round while the other waves wait at the barrier
     constexpr int TS = VS<MASK>::NV > 4 ? 128 : NTHR1 - 13;
     ks->sweep1d = [](const SweepArgs& a, int nb, hipStream_t s) {
+        // HLLD's short divisions shorten a workgroup's chain and leave a SIMD
+        // one or two waves: beyond two workgroups per CU the general form, with
+        // its third wave, is faster.  1601-cell tubes (13 tiles each), us a step,
+        // short / general: PPM 32 tubes 60.9 / 64.4, 48 86.7 / 82.1, 256 297 /
+        // 272; WENO5 32 65.9 / 69.9, 48 91.3 / 88.8, 256 327 / 298 (before the
+        // short form 318; WENO7 keeps it, 256 408 / 427).
+        constexpr int SHORT_BLOCKS = 512;
+        if constexpr (std::is_same<R, double>::value && !SPLIT && SOLVER == HLLD && (RECON == PPM || RECON == WENO5))
+            if (nb > SHORT_BLOCKS)
+                return launch_sweep(sweep1d_kernel<R, MASK, RECON, SOLVER, TS, SPLIT, AUTH, false>, a, nb, s, NTHR1);
         launch_sweep(sweep1d_kernel<R, MASK, RECON, SOLVER, TS, SPLIT, AUTH>, a, nb, s, NTHR1);
     };
     ks->ts1 = TS;

@@ -596,7 +596,7 @@ struct LineAcc {
     }
 };
 
-template <class R, int MASK, int RECON, int SOLVER, int TS, bool SPLIT = false, int AUTH = AUTH_MC>
+template <class R, int MASK, int RECON, int SOLVER, int TS, bool SPLIT = false, int AUTH = AUTH_MC, bool SHORT = true>
 __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
     static_assert(!SPLIT || sizeof(R) == 8, "split path keeps FP64 values");
     using V = VS<MASK>;
@@ -605,12 +605,12 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
     // interface states in fd's range are solved in its arithmetic (wave-uniform
     // choice): 192 ragged PPM/HLLC problems 1.81 -> 1.76 ms per 16 steps.
     // HLLD in fd takes 238-261 registers where the general form takes 134-150.
-    // PPM and WENO5 gain all the same (four 1601-cell tubes 45.8 -> 43.8 and
-    // 47.9 -> 45.7 us a step, 32 tubes 63.4 -> 60.5 and 69.3 -> 65.5, 64 tubes
-    // 102.5 -> 104.0 and 111.8 -> 113.6); PLM and WENO3, whose other phases are
-    // shorter, gain 2-4 % on a few tubes and lose up to 44 % on many (PLM, 64
-    // tubes, us a step: general 73.4, fd 104.9; WENO3 out of fd's range 98.7, 109.5)
-    constexpr bool FAST = std::is_same<R, double>::value && !SPLIT && RECON != PCM &&
+    // PPM and WENO5 gain all the same on few tubes (SHORT: the launch takes the
+    // other instantiation on many), WENO7 on any; PLM and WENO3, whose other
+    // phases are shorter, gain 2-4 % on a few tubes and lose up to 44 % on many
+    // (PLM, 64 tubes, us a step: general 73.4, fd 104.9; WENO3 out of fd's range
+    // 98.7, 109.5)
+    constexpr bool FAST = SHORT && std::is_same<R, double>::value && !SPLIT && RECON != PCM &&
                           (V::MHD ? SOLVER == HLLD && RECON != PLM && RECON != WENO3 : (SOLVER == LLF || SOLVER == HLLC));
     constexpr int HW_L = 5, HW_R = 6;                 // wS window [s0-5, s0+TS+6)
     constexpr int NQ = TS + HW_L + HW_R + 2;           // q window [s0-6, s0+TS+7)

@@ -600,3 +600,39 @@ def test_any_adiabatic_index_takes_the_arithmetic_it_needs(shape, solver, gamma)
             assert np.nanmax(np.abs(f[..., c] - h[..., c]), initial=0.) <= 1e-13 * top, (ax, c)
         e, w = got[ax]["eigmax"], want[ax]["eigmax"]
         assert (np.isnan(e) and np.isnan(w)) or abs(e - w) <= 1e-13 * w, (e, w)
+
+
+@pytest.mark.parametrize("subgrid,boundary", [("ppm", "edge"), ("weno5", "wrap")])
+def test_many_tubes_keep_the_bits_of_each(subgrid, boundary):
+    """1D HLLD of more tubes than two workgroups per CU, in the general
+    divisions, against each kind of tube alone, in the short ones."""
+    import torch
+    from astrea_amd.plan import Plan
+    n = [130, 700, 1601, 257]
+    tubes = []
+    for i, m in enumerate(n):
+        x = np.arange(m) / m
+        g = np.zeros((m, 8))
+        g[:, 0] = 1 + .1 * np.sin(7 * x + i)
+        g[:, 1:4] = g[:, :1] * np.stack([.2 * np.cos(5 * x), .1 * np.sin(9 * x), .1 + 0 * x], 1)
+        g[:, 5:] = np.stack([.75 + 0 * x, .3 * np.cos(6 * x), .2 * np.sin(8 * x)], 1)
+        g[:, 4] = (1 + .1 * np.cos(4 * x)) / .4 + .5 * (g[:, 1:4] ** 2).sum(1) / g[:, 0] + .5 * (g[:, 5:] ** 2).sum(1)
+        tubes.append(torch.from_numpy(g).cuda())
+
+    def run(which):
+        plan = Plan(1, subgrid, "hlld", "ssprk(3,3)",
+                    [dict(n0=n[i], boundary=boundary, dx=1 / n[i], gamma=1.4, cfl=.4, t_end=1e9) for i in which],
+                    varmask=0xFF)
+        plan.load([tubes[i] for i in which])
+        plan.reset()
+        plan.step(3)
+        out, st, offs = plan.state.clone(), plan.status(), plan.offsets + [plan.total]
+        plan.close()
+        assert bool(torch.isfinite(out).all()) and not any(s["failed"] for s in st)
+        return [out[:, offs[k]:offs[k + 1]] for k in range(len(which))], st
+    which = [i % 4 for i in range(100)]  # 25 x (2 + 6 + 13 + 3) tiles
+    both, st = run(which)
+    for i in range(4):
+        (one,), (s1,) = run([i])
+        for k in (i, 96 + i):
+            assert torch.equal(both[k], one) and st[k] == s1

@@ -63,3 +63,15 @@ def test_registers_leave_room_for_the_waves(kernel, mask, recons, last, waves):
         used = k[".vgpr_count"]  # accumulation registers included: one file of 512 per lane, in eights
         assert 512 // (used + 7 & ~7) >= waves and k[".vgpr_spill_count"] == 0, (name, used, k[".vgpr_spill_count"])
     assert found >= len(recons) * len(last)
+
+
+@pytest.mark.parametrize("recon", [PPM, WENO5])
+def test_hlld_of_many_tubes_leaves_room_for_three_waves(recon):
+    """The 1D HLLD sweep that a launch of more than two workgroups per CU takes
+    has the general divisions, whose registers leave room for a third wave."""
+    if not os.path.exists(L.LIB_PATH):
+        pytest.skip("library not built (run python -m astrea_amd._build)")
+    found = [k for name, k in _kernels().items()
+             if re.match(rf"_ZN2ah14sweep1d_kernelIdLi{ALL}ELi{recon}ELi{HLLD}ELi\d+ELb0ELi0ELb0E", name)]
+    assert len(found) == 1
+    assert 512 // (found[0][".vgpr_count"] + 7 & ~7) >= 3 and found[0][".vgpr_spill_count"] == 0
