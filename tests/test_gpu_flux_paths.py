@@ -636,3 +636,139 @@ def test_many_tubes_keep_the_bits_of_each(subgrid, boundary):
         (one,), (s1,) = run([i])
         for k in (i, 96 + i):
             assert torch.equal(both[k], one) and st[k] == s1
+
+
+def _hlld_keeps_the_short_form(g):
+    """Whether HLLD of neighbouring cells' states along the first axis (gamma =
+    1.4) stays in the short divisions' range: star densities positive, the
+    fast speeds' discriminants not negative, divisors not tiny."""
+    rho = g[..., 0]
+    u, b = g[..., 1:4] / rho[..., None], g[..., 5:8]
+    p = .4 * (g[..., 4] - .5 * rho * (u ** 2).sum(-1) - .5 * (b ** 2).sum(-1))
+    cs2, ca2, cax2 = 1.4 * p / rho, (b ** 2).sum(-1) / rho, b[..., 0] ** 2 / rho
+    disc = (cs2 + ca2) ** 2 - 4 * cs2 * cax2
+    cf = np.sqrt(.5 * (cs2 + ca2 + np.sqrt(np.maximum(disc, 0))))
+    left, right = slice(None, -1), slice(1, None)
+    rl, rr, ul, ur = rho[left], rho[right], u[left][..., 0], u[right][..., 0]
+    lo, c = np.minimum(ul, ur), np.maximum(cf[left], cf[right])
+    sl, sr = lo - c, lo + c
+    bl, br = .5 * (b[left] ** 2).sum(-1), .5 * (b[right] ** 2).sum(-1)
+    den = rl * (sl - ul) - rr * (sr - ur)
+    sm = (p[right] - p[left] + rl * ul * (sl - ul) - rr * ur * (sr - ur) + br - bl) / den
+    rls, rrs = rl * (sl - ul) / (sl - sm), rr * (sr - ur) / (sr - sm)
+    return (disc[left] >= 0) & (disc[right] >= 0) & (rls > 2. ** -90) & (rrs > 2. ** -90) & (np.abs(den) > 2. ** -90)
+
+
+@pytest.mark.parametrize("shape,subgrid,boundary", [((128,), "ppm", "wrap"), ((300,), "ppm", "wrap"),
+                                                    ((700, 640), "ppm", "wrap"), ((640, 700), "plm", "edge")], ids=str)
+def test_short_hlld_of_weak_waves_gives_the_general_bits(shape, subgrid, boundary):
+    """As for strong shocks above, where nearly every wave of 64 lanes is solved
+    in the general form after all: here the waves are weak, so that the state of
+    order one stays in the short form, as its range evaluated on the host shows
+    (1D, and the marching launch in 2D)."""
+    from astrea_amd.plan import Plan
+    dims = len(shape)
+    if dims == 2:
+        base = _smooth(shape, 3, mhd=True)
+    else:
+        base = _smooth(shape + (1,), 3, mhd=True)[:, 0]
+        x = 2 * np.pi * np.arange(shape[0]) / shape[0]
+        base[..., 3] = base[..., 0] * .1 * np.cos(x)
+        base[..., 5], base[..., 7] = .75, .2 * np.sin(x)
+        base[..., 4] += .7
+    assert _hlld_keeps_the_short_form(base).all()
+    if dims == 2:
+        swap = base.swapaxes(0, 1)[..., [0, 2, 1, 3, 4, 6, 5, 7]]
+        assert _hlld_keeps_the_short_form(swap).all()
+    names = (0, 1, 2, 3, 5, 6, 7) if dims == 1 else (0, 1, 2, 5, 6)
+
+    def fluxes(g):
+        plan = Plan(dims, subgrid, "hlld", "ssprk(3,3)",
+                    [dict(n0=shape[0], n1=shape[1] if dims == 2 else 1, boundary=boundary, dx=1 / 64, gamma=1.4, cfl=.4,
+                          t_end=1e9)], varmask=0xFF if dims == 1 else 0x77, magnetic_2d=dims == 2, compat="physical")
+        plan.load([g])
+        out = [plan.evolve_space(parity=q) for q in (0, 1)]
+        plan.close()
+        return out
+    ref, got = fluxes(base), fluxes(np.ldexp(base, [0] + 3 * [-60] + [-120] + 3 * [-60]))
+    for q in (0, 1):
+        for ax in range(dims):
+            f, g = ref[q][ax]["flux"], got[q][ax]["flux"]
+            assert np.isfinite(f).all()
+            for i in names:
+                assert np.array_equal(g[..., i], np.ldexp(f[..., i], [0, -60, -60, -60, 0, -60, -60, -60][i] - 60)), (q, ax, i)
+
+
+@pytest.mark.parametrize("subgrid,solver,boundary", [("ppm", "hllc", "wrap"), ("plm", "hllc", "edge"), ("weno5", "llf", "edge")])
+def test_one_cell_outside_the_short_range_at_a_marching_size(subgrid, solver, boundary):
+    """A transverse velocity of 2^-120 in one cell of a gas otherwise at rest
+    across takes the lines that see it out of the short range, and only those:
+    the marching launch against the 2D tiles, bit for bit."""
+    import torch
+    from astrea_amd.plan import Plan
+    from tests.test_zz_no_alloc import _static_call
+    g = _smooth((700, 640), 5)
+    g[..., 4] -= .5 * g[..., 2] ** 2 / g[..., 0]
+    g[..., 2] = 0.
+    for at in ((333, 211), (0, 639)):
+        g[at][2] = g[at][0] * 2. ** -120
+    plan = Plan(2, subgrid, solver, "ssprk(3,3)",
+                [dict(n0=700, n1=640, boundary=boundary, dx=1 / 512, gamma=1.4, cfl=.4, t_end=1e9)], varmask=0x17)
+    plan.load([torch.from_numpy(g).cuda()])
+    for parity in (0, 1):
+        ref = plan.evolve_space(parity)
+        rc, f0, f1, eig = _static_call(plan, parity)
+        assert rc == 0
+        assert bool(torch.isfinite(ref[0]["raw"]).all()) and bool(torch.isfinite(ref[1]["raw"]).all())
+        assert torch.equal(f0, ref[0]["raw"]) and torch.equal(f1, ref[1]["raw"])
+        assert eig == [ref[0]["eigmax"], ref[1]["eigmax"]]
+    plan.close()
+
+
+@pytest.mark.parametrize("subgrid,boundary", [("plm", "edge"), ("ppm", "wrap"), ("weno5", "edge"), ("weno5", "wrap")])
+@pytest.mark.parametrize("shape", [(700, 640), (640, 505)], ids=str)
+def test_marching_hlld_against_the_oracle(shape, subgrid, boundary):
+    """HLLD fluxes and wave speeds of a grid large enough for the marching
+    launch against the oracle's: 1e-13 of each component's largest flux, some
+    450 units in the last place."""
+    from astrea_amd.plan import Plan
+    from oracle import astrea_oracle as O
+    g = _smooth(shape, 9, mhd=True)
+    plan = Plan(2, subgrid, "hlld", "ssprk(3,3)",
+                [dict(n0=shape[0], n1=shape[1], boundary=boundary, dx=1 / 512, gamma=1.4, cfl=.4, t_end=1e9)],
+                varmask=0x77, magnetic_2d=True)
+    plan.load([g])
+    got = plan.evolve_space(0)
+    plan.close()
+    want = O.evolve_space(g, O.Scheme(dimension=2, subgrid=subgrid, solver="hlld", boundary=boundary, gamma=1.4, cfl=.4,
+                                      dx=1 / 512, magnetic_2d=True))
+    for ax in (0, 1):
+        f, h = got[ax]["flux"], want[ax]["flux"]
+        assert np.isfinite(f).all()
+        for c in range(8):
+            assert np.abs(f[..., c] - h[..., c]).max() <= 1e-13 * np.abs(h[..., c]).max(), (ax, c)
+        assert abs(got[ax]["eigmax"] - want[ax]["eigmax"]) <= 1e-13 * want[ax]["eigmax"]
+
+
+@pytest.mark.parametrize("flattener", ["off", "astrea"])
+@pytest.mark.parametrize("boundary", ["wrap", "edge"])
+@pytest.mark.parametrize("shapes", [((31, 9), (32, 8), (33, 7)), ((64, 4), (65, 5), (63, 3)), ((2, 3), (97, 130))], ids=str)
+def test_shared_faces_of_smooth_states_match_each_cell_for_itself(shapes, boundary, flattener):
+    """As above with a state that stays finite for the three steps, which are
+    compared as they are."""
+    import torch
+    from astrea_amd.plan import Plan
+    probs = [dict(n0=a, n1=b, boundary=boundary, dx=1 / max(a, b), gamma=1.4, cfl=.3, t_end=1e9) for a, b in shapes]
+    grids = [torch.from_numpy(_smooth(s, 21 + i)).cuda() for i, s in enumerate(shapes)]
+    outs = []
+    for fuse in (False, True):
+        plan = Plan(2, "ppm", "hllc", "ssprk(3,3)", probs, varmask=0x17, flattener=flattener, compat="physical",
+                    fuse2d=fuse)
+        plan.load(grids)
+        plan.reset()
+        plan.step(3)
+        outs.append((plan.state.clone(), plan.status()))
+        plan.close()
+    assert bool(torch.isfinite(outs[0][0]).all()) and not any(s["failed"] for s in outs[0][1])
+    assert torch.equal(outs[0][0], outs[1][0])
+    assert outs[0][1] == outs[1][1]
