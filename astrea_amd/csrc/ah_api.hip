@@ -193,6 +193,7 @@ struct ah_plan {
     // flux lists, of the same problems at any time: a captured step keeps its
     // kernel, whichever form the plan launches by then.
     TileList tl[10];
+    std::vector<char> listed;    // per problem: its tiles are in the device lists (empty: not known)
     int cus = 256;
     bool march = false;          // the flux launches take the marching form
     int max_blocks = 8192;  // grid cap per launch (workgroups loop over the tiles beyond it)
@@ -427,6 +428,7 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
         case AH_SSPRK104: p->nregs = sch->magnetic_2d ? 4 : 3; break;  // + the refined increment
     }
     p->cus = cus;
+    p->listed.assign(nprob, 1);
     // problem tables and tiles
     std::vector<ProbDesc> pd(nprob);
     // combination tiles: 256 cells (one per thread) in 1D, so the few large
@@ -519,11 +521,13 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
         if (!up) break;
         L.count = (int)L.full.size();
         if (!L.count && (&L == p->tl + 3 || &L == p->tl + 4 || &L >= p->tl + 8)) continue;  // a flux form not launched
+        // (the tiles beside marching lists are first copied when the plan turns to them: ah_plan_compact)
+        const bool now = !(p->march && (&L == p->tl + 3 || &L == p->tl + 4));
         up = hipMalloc((void**)&L.d_count, sizeof(int)) == hipSuccess &&
-             hipMemcpy(L.d_count, &L.count, sizeof(int), hipMemcpyHostToDevice) == hipSuccess;
+             (!now || hipMemcpy(L.d_count, &L.count, sizeof(int), hipMemcpyHostToDevice) == hipSuccess);
         if (up && L.count)
             up = hipMalloc((void**)&L.d, std::max(L.full.size(), L.room) * sizeof(Tile)) == hipSuccess &&
-                 hipMemcpy(L.d, L.full.data(), L.full.size() * sizeof(Tile), hipMemcpyHostToDevice) == hipSuccess;
+                 (!now || hipMemcpy(L.d, L.full.data(), L.full.size() * sizeof(Tile), hipMemcpyHostToDevice) == hipSuccess);
     }
     // 32 workgroups per CU: a 1024^2 grid's sweeps then launch one workgroup
     // per tile and the hardware balances the last round (2048 persistent
@@ -651,13 +655,20 @@ int ah_plan_reset(ah_plan* p, void* stream) {
     if (!p) return AH_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
     HIPCHK(hipStreamSynchronize(s));
-    for (TileList& L : p->tl) {  // every problem is active again: full work lists
-        if (L.full.empty()) continue;
-        L.count = (int)L.full.size();
-        HIPCHK(hipMemcpy(L.d, L.full.data(), L.full.size() * sizeof(Tile), hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(L.d_count, &L.count, sizeof(int), hipMemcpyHostToDevice));
+    // every problem is active again: full work lists, if the device holds others
+    // (two copies a list, each waited for: 15 us and more)
+    const std::vector<char> all(p->nprob, 1);
+    if (p->listed != all) {
+        p->listed.clear();
+        for (TileList& L : p->tl) {
+            if (L.full.empty()) continue;
+            L.count = (int)L.full.size();
+            HIPCHK(hipMemcpy(L.d, L.full.data(), L.full.size() * sizeof(Tile), hipMemcpyHostToDevice));
+            HIPCHK(hipMemcpy(L.d_count, &L.count, sizeof(int), hipMemcpyHostToDevice));
+        }
+        p->listed = all;
+        p->march = !p->tl[8].full.empty();
     }
-    p->march = !p->tl[8].full.empty();
     hipLaunchKernelGGL(reset_kernel, dim3((p->nprob + 255) / 256), dim3(256), 0, s, p->d_pd, p->d_ps, p->nprob);
     HIPCHK(hipGetLastError());
     return AH_OK;
@@ -1105,8 +1116,14 @@ int ah_plan_compact(ah_plan* p, int* nactive, void* stream) {
     HIPCHK(hipMemcpyAsync(h.data(), p->d_ps, p->nprob * sizeof(ProbState), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     int na = 0;
-    for (const ProbState& q : h) na += q.active ? 1 : 0;
+    std::vector<char> active;
+    for (const ProbState& q : h) {
+        active.push_back(q.active ? 1 : 0);
+        na += active.back();
+    }
     if (nactive) *nactive = na;
+    if (active == p->listed) return AH_OK;
+    p->listed.clear();
     // The marching lists are split anew for the problems left, and the 2D tiles
     // take over where they are the faster form: in tiles of the lines that suit
     // a large problem, the small ones it leaves behind are a few long waves.
@@ -1114,12 +1131,13 @@ int ah_plan_compact(ah_plan* p, int* nactive, void* stream) {
     // lines, 155 so; six 400^2 MHD ones down to one 1160, 587.  The first
     // step graph after the turn is a new one, 0.3 ms for 16 steps.
     FluxForm form;
+    bool march = p->march;
     if (!p->tl[8].full.empty() && na > 0) {
         std::vector<const ah_problem*> left;
         for (int i = 0; i < p->nprob; ++i)
             if (h[i].active) left.push_back(&p->probs[i]);
         form = flux_form(p->sch, p->ks, p->cus, left);
-        p->march = form.march || p->tl[3].full.empty();
+        march = form.march || p->tl[3].full.empty();
     }
     for (int l = 0; l < 10; ++l) {
         TileList& L = p->tl[l];
@@ -1137,6 +1155,8 @@ int ah_plan_compact(ah_plan* p, int* nactive, void* stream) {
         if (L.count) HIPCHK(hipMemcpy(L.d, act.data(), act.size() * sizeof(Tile), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(L.d_count, &L.count, sizeof(int), hipMemcpyHostToDevice));
     }
+    p->listed = active;
+    p->march = march;
     return AH_OK;
 }
 
