@@ -176,10 +176,6 @@ struct DivDx {
 // result cannot change what is computed from it, and where a NaN operand can
 // only come from a NaN cell of the stencil, whose own interface states are
 // NaN through the arithmetic, so that the step fails as numpy's does.
-__device__ inline double hmin(double a, double b) { return __builtin_fmin(a, b); }
-__device__ inline float hmin(float a, float b) { return __builtin_fminf(a, b); }
-__device__ inline double hmax(double a, double b) { return __builtin_fmax(a, b); }
-__device__ inline float hmax(float a, float b) { return __builtin_fmaxf(a, b); }
 // The instructions themselves, plain and of absolute values: the compiler's
 // fmin/fmax first quiet each operand it has not just computed, one more
 // instruction apiece.
@@ -203,12 +199,10 @@ __device__ inline double imax_abs(double a, double b) {
     asm("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
-__device__ inline float imin(float a, float b) { return hmin(a, b); }
-__device__ inline float imax(float a, float b) { return hmax(a, b); }
-__device__ inline float imin_abs(float a, float b) { return hmin(ah_fabs(a), ah_fabs(b)); }
-__device__ inline float imax_abs(float a, float b) { return hmax(ah_fabs(a), ah_fabs(b)); }
-__device__ inline double ah_copysign(double m, double s) { return __builtin_copysign(m, s); }
-__device__ inline float ah_copysign(float m, float s) { return __builtin_copysignf(m, s); }
+__device__ inline float imin(float a, float b) { return __builtin_fminf(a, b); }
+__device__ inline float imax(float a, float b) { return __builtin_fmaxf(a, b); }
+__device__ inline float imin_abs(float a, float b) { return __builtin_fminf(ah_fabs(a), ah_fabs(b)); }
+__device__ inline float imax_abs(float a, float b) { return __builtin_fmaxf(ah_fabs(a), ah_fabs(b)); }
 __device__ inline fd nmin(fd a, fd b) { return fd(imin(a.v, b.v)); }
 __device__ inline fd nmax(fd a, fd b) { return fd(imax(a.v, b.v)); }
 template <class R>
