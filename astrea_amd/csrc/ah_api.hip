@@ -434,7 +434,12 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
     // combination tiles: 256 cells (one per thread) in 1D, so the few large
     // problems left at the end of an ensemble still spread over many CUs, and
     // in 2D up to 128^2, whose 64 tiles still end the step themselves (below);
-    // 1024 beyond, where four cells per thread ran faster on 1024^2 grids
+    // 1024 beyond, where four cells per thread run faster on large grids.  us a
+    // step of one grid alone in tiles of 1024 / 256 cells: PLM/HLLC SSPRK(3,3)
+    // 136^2 94 / 90, 256^2 116 / 112, 512^2 231 / 228, 700^2 336 / 338, 1000^2
+    // 488 / 493; WENO5/HLLC RK4 256^2 193 / 182, 512^2 387 / 383, 700^2 577 /
+    // 577, 1000^2 909 / 919.  (A lone grid of 128^2 to 512^2 would still gain
+    // 1-6 % by the small tiles; problems of that size in numbers were not timed.)
     long long most_cells = 0;
     for (int i = 0; i < nprob; ++i) most_cells = std::max(most_cells, (long long)probs[i].n0 * std::max(probs[i].n1, 1));
     p->comb_cells = sch->dims == 1 || most_cells <= 64 * 256 ? 256 : 1024;

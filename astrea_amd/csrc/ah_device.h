@@ -976,6 +976,126 @@ __device__ inline V8<R> flux_hlld(const Iface<R>& s, R Bn, R gamma, bool* ok) {
     } else return hlld_flux<R, MASK, SAX>(h, Bn, s.qm, s.qp, s.fm, s.fp);
 }
 
+// The waves and flux of split precision, whose units contract multiplications
+// into additions: both sides whole, the side of the contact selected last.
+// Another order of operations contracts otherwise, and where a field along the
+// axis makes HLLD's divisors vanish the last bits decide how long a run lasts
+// (160 x 130 cells PPM: 12 steps so, 10 with the energies of one side).
+template <int MASK, int SAX>
+__device__ inline V8<double> flux_hlld_split(const Iface<double>& s, double Bn, double gamma) {
+    using R = double;
+    constexpr int A = SAX % 3, O = (SAX + 1) % 3, C = (SAX + 2) % 3;
+    auto cfast = [&](const V8<R>& w) {
+        const R rho = w.c[0], p = w.c[4];
+        const R cs = ah_sqrt(gdiv(gamma * p, rho));
+        const R ca = gdiv(ah_sqrt((w.c[5] * w.c[5] + w.c[6] * w.c[6]) + w.c[7] * w.c[7]), ah_sqrt(rho));
+        const R cax = gdiv(w.c[5], ah_sqrt(rho));
+        const R cs2 = cs * cs, ca2 = ca * ca;
+        return ah_sqrt(R(0.5) * (cs2 + ca2 + ah_sqrt(sq(cs2 + ca2) - R(4) * cs2 * (cax * cax))));
+    };
+    auto n2 = [](R a, R b, R c) {
+        R n = ah_sqrt((a * a + b * b) + c * c);
+        return n * n;
+    };
+    auto d3 = [](R a0, R b0, R a1, R b1, R a2, R b2) { return (a0 * b0 + a1 * b1) + a2 * b2; };
+    const V8<R>&wL = s.wm, &wR = s.wp, &QL = s.qm, &QR = s.qp;
+    const R rhoL = wL.c[0], pL = wL.c[4], rhoR = wR.c[0], pR = wR.c[4];
+    const R uL = wL.c[SAX + 1], uR = wR.c[SAX + 1];
+    const R cfL = cfast(wL), cfR = cfast(wR);
+    const R umin = nmin(uL, uR), cmax = nmax(cfL, cfR);
+    const R sL = umin - cmax, sR = umin + cmax;
+    const R bL2 = n2(wL.c[5], wL.c[6], wL.c[7]), bR2 = n2(wR.c[5], wR.c[6], wR.c[7]);
+    const R den = rhoL * (sL - uL) - rhoR * (sR - uR);
+    const R sM = gdiv(pR - pL + rhoL * uL * (sL - uL) - rhoR * uR * (sR - uR) + R(0.5) * bR2 - R(0.5) * bL2, den);
+    const R rLs = rhoL * gdiv(sL - uL, sL - sM), rRs = rhoR * gdiv(sR - uR, sR - sM);
+    const R sLs = sM - gdiv(wL.c[SAX + 5], ah_sqrt(rLs)), sRs = sM - gdiv(wR.c[SAX + 5], ah_sqrt(rRs));
+    const R ps = gdiv(rhoL * (pR + R(0.5) * bR2) * (sL - uL) - rhoR * (pL + R(0.5) * bL2) * (sR - uR) +
+                          rhoR * rhoL * (sL - uL) * (sR - uR),
+                      den);
+    const R Bn2 = Bn * Bn;
+    const R dL = rhoL * (sL - uL) * (sL - sM) - Bn2, dR = rhoR * (sR - uR) * (sR - sM) - Bn2;
+    const R vyLs = wL.c[O + 1] - Bn * wL.c[O + 5] * gdiv(sM - uL, dL);
+    const R vyRs = wR.c[O + 1] - Bn * wR.c[O + 5] * gdiv(sM - uR, dR);
+    const R vzLs = wL.c[C + 1] - Bn * wL.c[C + 5] * gdiv(sM - uL, dL);
+    const R vzRs = wR.c[C + 1] - Bn * wR.c[C + 5] * gdiv(sM - uR, dR);
+    const R ByLs = wL.c[O + 5] * gdiv(rhoL * sq(sL - uL) - Bn2, dL);
+    const R ByRs = wR.c[O + 5] * gdiv(rhoR * sq(sR - uR) - Bn2, dR);
+    const R BzLs = wL.c[C + 5] * gdiv(rhoL * sq(sL - uL) - Bn2, dL);
+    const R BzRs = wR.c[C + 5] * gdiv(rhoR * sq(sR - uR) - Bn2, dR);
+    V8<R> QLs, QRs;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) QLs.c[i] = QRs.c[i] = R(0);
+    QLs.c[0] = rLs;
+    QRs.c[0] = rRs;
+    QLs.c[A + 1] = rhoL * sM;
+    QRs.c[A + 1] = rhoR * sM;
+    QLs.c[O + 1] = rhoL * vyLs;
+    QRs.c[O + 1] = rhoR * vyRs;
+    QLs.c[C + 1] = rhoL * vzLs;
+    QRs.c[C + 1] = rhoR * vzRs;
+    QLs.c[A + 5] = QL.c[A + 5];
+    QRs.c[A + 5] = QR.c[A + 5];
+    QLs.c[O + 5] = ByLs;
+    QRs.c[O + 5] = ByRs;
+    QLs.c[C + 5] = BzLs;
+    QRs.c[C + 5] = BzRs;
+    const R vBL = d3(wL.c[1], wL.c[5], wL.c[2], wL.c[6], wL.c[3], wL.c[7]);
+    const R vBR = d3(wR.c[1], wR.c[5], wR.c[2], wR.c[6], wR.c[3], wR.c[7]);
+    const R mBLs = d3(QLs.c[1], QLs.c[5], QLs.c[2], QLs.c[6], QLs.c[3], QLs.c[7]);
+    const R mBRs = d3(QRs.c[1], QRs.c[5], QRs.c[2], QRs.c[6], QRs.c[3], QRs.c[7]);
+    QLs.c[4] = gdiv(QL.c[4] * (sL - uL) - uL * (pL + R(0.5) * bL2) + ps * sM + Bn * (vBL - mBLs), sL - sM);
+    QRs.c[4] = gdiv(QR.c[4] * (sR - uR) - uR * (pR + R(0.5) * bR2) + ps * sM + Bn * (vBR - mBRs), sR - sM);
+    const R sg = nsign(Bn);
+    const R srL = ah_sqrt(rLs), srR = ah_sqrt(rRs), srs = srL + srR, srp = ah_sqrt(rRs * rLs);
+    const R vyss = gdiv(vyRs * srR + vyLs * srL + sg * (ByLs - ByRs), srs);
+    const R vzss = gdiv(vzRs * srR + vzLs * srL + sg * (BzLs - BzRs), srs);
+    const R Byss = gdiv(ByLs * srR + ByRs * srL + sg * (vyLs - vyRs) * srp, srs);
+    const R Bzss = gdiv(BzLs * srR + BzRs * srL + sg * (vzLs - vzRs) * srp, srs);
+    V8<R> QLss, QRss;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) QLss.c[i] = QRss.c[i] = R(0);
+    QLss.c[0] = rLs;
+    QRss.c[0] = rRs;
+    QLss.c[A + 1] = sM;
+    QRss.c[A + 1] = sM;
+    QLss.c[O + 1] = vyss;
+    QRss.c[O + 1] = vyss;
+    QLss.c[C + 1] = vzss;
+    QRss.c[C + 1] = vzss;
+    QLss.c[A + 5] = QLs.c[A + 5];
+    QRss.c[A + 5] = QRs.c[A + 5];
+    QLss.c[O + 5] = Byss;
+    QRss.c[O + 5] = Byss;
+    QLss.c[C + 5] = Bzss;
+    QRss.c[C + 5] = Bzss;
+    const R mBLss = d3(QLss.c[1], QLss.c[5], QLss.c[2], QLss.c[6], QLss.c[3], QLss.c[7]);
+    const R mBRss = d3(QRss.c[1], QRss.c[5], QRss.c[2], QRss.c[6], QRss.c[3], QRss.c[7]);
+    QLss.c[4] = QLs.c[4] - srL * sg * (mBLs - mBLss);
+    QRss.c[4] = QRs.c[4] - srR * sg * (mBRs - mBRss);
+    // region select (solvers.py:226-231), later masks overwrite earlier ones
+    int reg = 0;  // 0: F(w-)
+    if ((sL <= R(0)) && (R(0) < sLs)) reg = 1;
+    if ((sLs <= R(0)) && (R(0) < sM)) reg = 2;
+    if ((sM <= R(0)) && (R(0) < sRs)) reg = 3;
+    if ((sRs <= R(0)) && (R(0) <= sR)) reg = 4;
+    if (sR < R(0)) reg = 5;
+    V8<R> F;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        R v;
+        switch (reg) {
+            case 1: v = s.fm.c[i] + (QLs.c[i] - QL.c[i]) * sL; break;
+            case 2: v = s.fm.c[i] + (QLss.c[i] - QLs.c[i]) * sLs; break;
+            case 3: v = s.fp.c[i] + (QRss.c[i] - QRs.c[i]) * sRs; break;
+            case 4: v = s.fp.c[i] + (QRs.c[i] - QR.c[i]) * sR; break;
+            case 5: v = s.fp.c[i]; break;
+            default: v = s.fm.c[i]; break;
+        }
+        F.c[i] = v;
+    }
+    return F;
+}
+
 // ---- Osher-Solomon flux with the Dumbser-Toro path integral (solvers.py:236-284)
 namespace dots {
 // 3-point Gauss-Legendre on [0, 1] as the reference builds them

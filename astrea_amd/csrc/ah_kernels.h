@@ -528,8 +528,11 @@ __device__ inline V8<R> riemann(const Iface<R>& s, R lam, int sax, R Bn, R gamma
         return flux_dots<MASK>(s, sax, gamma);
     else if constexpr (SOLVER == ES)
         return flux_es<MASK>(s, sax, gamma);
-    else
+    else {
+        if constexpr (std::is_same<R, double>::value)
+            if (split) return sax == 0 ? flux_hlld_split<MASK, 0>(s, Bn, gamma) : flux_hlld_split<MASK, 1>(s, Bn, gamma);
         return sax == 0 ? flux_hlld<R, MASK, 0>(s, Bn, gamma, ok) : flux_hlld<R, MASK, 1>(s, Bn, gamma, ok);
+    }
 }
 
 // Osher-Solomon: a non-finite flux marks the step failed (flux_dots returns
