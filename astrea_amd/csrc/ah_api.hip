@@ -196,6 +196,7 @@ struct ah_plan {
     std::vector<char> listed;    // per problem: its tiles are in the device lists (empty: not known)
     int cus = 256;
     bool march = false;          // the flux launches take the marching form
+    bool many = false;           // the largest problem has many sweep tiles (many_tiles)
     int max_blocks = 8192;  // grid cap per launch (workgroups loop over the tiles beyond it)
     // captured step graphs (ah_plan_step_graph), one for each form of the flux launches
     hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
@@ -510,6 +511,7 @@ int ah_plan_create(const ah_scheme* sch, int nprob, const ah_problem* probs, ah_
         max_ctiles = std::max(max_ctiles, (cells + ct - 1) / ct);
     }
     p->total = total;
+    p->many = many_tiles(sch->dims, most_cells / (sch->dims == 1 ? p->ks.ts1 : p->ks.fts[0] * p->ks.ftt[0]));
     // each combination tile of the step's last combination counts itself on
     // its problem's counter; beyond a few dozen tiles per problem the atomics
     // on one address cost more than the separate end-of-step launch (1024^2:
@@ -703,7 +705,7 @@ static void launch_space(ah_plan* p, const double* X, double* Lout, int stage0, 
     a.X = X;
     a.xl = xl;
     a.stage_idx = stage_idx;
-    a.stage0 = stage0;
+    a.stage0 = stage0 && p->many ? 2 : stage0;
     a.parity_override = parity_override;
     if (fuse33) {
         a.fuse_k2 = p->regs[2];
@@ -1544,7 +1546,7 @@ int ah_evolve_space_static(const ah_scheme* sch, const ah_problem* q, int parity
     a.compat = sch->compat;
     a.av = sch->av;
     a.X = grid;
-    a.stage0 = 1;
+    a.stage0 = many_tiles(sch->dims, spec[nlists - 1].n) ? 2 : 1;
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
         hipDeviceProp_t prop;

@@ -75,7 +75,7 @@ struct SweepArgs {
     const Tile* tiles;
     int ntiles;             // tile count when ntiles_dev is null
     const int* ntiles_dev;  // device-resident tile count (compactable lists)
-    int stage0;   // accumulate the eigmax for dt (stage 0 of a step)
+    int stage0;   // accumulate the eigmax for dt (stage 0 of a step); 2: the largest problem has many tiles
     int limiter;  // PLM slope limiter
     int flattener;
     int parity_override;  // -1: use per-problem parity
@@ -559,24 +559,38 @@ __device__ inline void wave_max(double v, double* red) {
     }
     if ((threadIdx.x & 63) == 0) reinterpret_cast<unsigned long long*>(red)[threadIdx.x >> 6] = b;
 }
-__device__ inline void max_of_waves(unsigned long long* dst, const double* red) {
+// One address takes an atomic every 3 ns, and the tiles of a large grid come to
+// it together: with `look` each looks first, and most find as much there
+// already (the maximum only grows during a launch, so that an older value costs
+// an atomic and no more).  The look holds up a workgroup's end, so that few
+// tiles go without (many_tiles).  us a step of forward Euler, without / with it: 1D
+// PLM/HLLC 5000 cells (21 tiles) 9.6 / 10.0, 80 000 (330) 15.2 / 16.0, 120 000
+// (494) 17.9 / 17.0, 1 million 70 / 44; PLM/LLF 120 000 17.4 / 17.7, 160 000 (659)
+// 19.8 / 19.0; 2D tiles, PPM/LLF split 100^2 (70) 34.9 / 35.4, 300^2 (570) 50 / 54.5,
+// 400^2 (1000) 78 / 69.6, 1000^2 270 / 223; PLM/HLLC split 300^2 44 / 51, 400^2 71 /
+// 64; PCM/LLF 300^2 48 / 50, 400^2 68 / 64.5, 1000^2 228 / 195; PCM/HLLC 400^2 74 / 72,
+// 1000^2 240 / 235, 1400^2 444 / 450, which goes without.
+// (Counted on the host for the plan's largest problem: in the tile, the count
+// took the 2D HLLC kernels 60 registers and their third wave.)
+inline bool many_tiles(int dims, long long tiles) { return tiles > (dims == 1 ? 450 : 800); }
+__device__ inline void max_of_waves(unsigned long long* dst, const double* red, bool look) {
     const unsigned long long* r = reinterpret_cast<const unsigned long long*>(red);
     if (threadIdx.x == 0) {
         unsigned long long m = r[0];
         for (int i = 1; i < (int)(blockDim.x >> 6); ++i) m = r[i] > m ? r[i] : m;
-        // One address takes an atomic every 3 ns, and a large grid's tiles come to
-        // it together: most find as much there already.  The maximum only grows
-        // during a launch, so that an older value costs an atomic and no more.
-        // 2 million cells of 1D PLM/HLLC 107 -> 55 us a first stage, 700 000 of
-        // WENO3 47 -> 35 (whose other stages take 34).
-        if (m > __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(dst, m);
+        if (look) {
+            if (m > __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(dst, m);
+        } else if (m != 0ull) {
+            atomicMax(dst, m);
+        }
     }
 }
-__device__ inline void block_max_atomic(double v, unsigned long long* dst, double* red) {
+__device__ inline void block_max_atomic(double v, unsigned long long* dst, double* red, bool look) {
     wave_max(v, red);
     __syncthreads();
-    max_of_waves(dst, red);
+    max_of_waves(dst, red, look);
 }
+
 
 // ============================================================================
 // 1D: one fused kernel per stage: load -> cons->prim -> reconstruct/limit ->
@@ -904,7 +918,7 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
     }
     if constexpr (!MERGED) {
         if (bad) atomicOr(&ps->fail_flag, 1);
-        if (a.stage0) block_max_atomic(lmax, &ps->eig[0], red);
+        if (a.stage0) block_max_atomic(lmax, &ps->eig[0], red, a.stage0 > 1);
         __syncthreads();
     }
     // E: interface fluxes k in [s0, s0+TS]
@@ -1015,7 +1029,7 @@ __global__ __launch_bounds__(256) void sweep1d_kernel(SweepArgs a) {
     __syncthreads();
     // (its way to memory and back runs beside the differences)
     if constexpr (MERGED)
-        if (a.stage0) max_of_waves(&ps->eig[0], red);
+        if (a.stage0) max_of_waves(&ps->eig[0], red, a.stage0 > 1);
     // F: L = -(F[i+1] - F[i]) / dx (evolvers.py:41-60)
     const DivDx bydx(pd.dx);
     int hit_;
@@ -1675,7 +1689,7 @@ void flux2d_kernel(SweepArgs a) {
         }
     }
     if (bad) atomicOr(&ps->fail_flag, 1);
-    if (a.stage0) block_max_atomic(lmax, &ps->eig[AX], red);
+    if (a.stage0) block_max_atomic(lmax, &ps->eig[AX], red, !(CONV == 0 && SOLVER == HLLC) && a.stage0 > 1);
     __syncthreads();
     // C: q+-, f+- and the face-average flux on lines [t0-1, t0+TT+1)
     int xhit_;

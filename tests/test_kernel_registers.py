@@ -75,3 +75,15 @@ def test_hlld_of_many_tubes_leaves_room_for_three_waves(recon):
              if re.match(rf"_ZN2ah14sweep1d_kernelIdLi{ALL}ELi{recon}ELi{HLLD}ELi\d+ELb0ELi0ELb0E", name)]
     assert len(found) == 1
     assert 512 // (found[0][".vgpr_count"] + 7 & ~7) >= 3 and found[0][".vgpr_spill_count"] == 0
+
+
+def test_2d_flux_tiles_of_hllc_leave_room_for_three_waves():
+    """The 2D HLLC flux tiles of FP64 hydrodynamics, whose LDS lets three
+    workgroups share a CU, keep the registers for it."""
+    if not os.path.exists(L.LIB_PATH):
+        pytest.skip("library not built (run python -m astrea_amd._build)")
+    found = {name: k for name, k in _kernels().items()
+             if re.match(rf"_ZN2ah13flux2d_kernelIdLi{HYDRO2}ELi({LLF}|{HLLC})ELi[012]ELi[01]ELi16ELi10ELb0ELi256ELin1E", name)}
+    assert len(found) == 12
+    for name, k in found.items():
+        assert 512 // (k[".vgpr_count"] + 7 & ~7) >= 3 and k[".vgpr_spill_count"] == 0, (name, k[".vgpr_count"])
